@@ -7,6 +7,7 @@ raises.
 """
 import ctypes
 import os
+import struct
 
 import torch  # noqa: F401  (must precede the CDLL load, see module docstring)
 
@@ -61,15 +62,33 @@ class SegmentIO(ctypes.Structure):
 
 assert ctypes.sizeof(Tile) == 16
 
-_lib = None
 
-# (name, restype, argtypes) of every symbol include/dkv.h declares.
+def _layout(structure):
+    """struct.Struct of a ctypes Structure: one value per field (per element of an array field), its
+    own padding in between. Every field is a native int, float or address."""
+    codes = {ctypes.c_void_p: 'P', ctypes.c_int64: 'q', ctypes.c_int32: 'i', ctypes.c_float: 'f', ctypes.c_uint16: 'H',
+             ctypes.c_uint8: 'B'}
+    fmt = ''.join(codes[t] if t in codes else f'{t._length_}{codes[t._type_]}' for _, t in structure._fields_)
+    out = struct.Struct(fmt)
+    assert out.size == ctypes.sizeof(structure), structure
+    return out
+
+
+TILE, PACK_JOB, ATTN_ARGS = _layout(Tile), _layout(PackJob), _layout(AttnArgs)
+
+_lib = None
+_zeroed_workspace = False
+
+# (name, restype, argtypes) of every symbol include/dkv.h declares. The argument blocks of the calls
+# that run once per layer (dkv_pack, dkv_attend) are declared as addresses: a Structure by reference
+# or the bytes PACK_JOB / ATTN_ARGS make in one call, a fifth of the time of setting a Structure's
+# fields one by one.
 SIGNATURES = [
     ('dkv_version', ctypes.c_int, []),
     ('dkv_last_error', ctypes.c_char_p, []),
     ('dkv_subblock_bytes', ctypes.c_int64, [ctypes.c_int32, ctypes.c_int32]),
     ('dkv_slab_bytes', ctypes.c_int64, [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32]),
-    ('dkv_pack', ctypes.c_int, [ctypes.POINTER(PackJob), ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
+    ('dkv_pack', ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
                                 ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p]),
     ('dkv_pack_batch', ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p,
                                       ctypes.c_int64, ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32,
@@ -79,8 +98,8 @@ SIGNATURES = [
     ('dkv_reconstruct', ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32,
                                        ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p,
                                        ctypes.c_int32, ctypes.c_void_p]),
-    ('dkv_attend_workspace_bytes', ctypes.c_int64, [ctypes.POINTER(AttnArgs)]),
-    ('dkv_attend', ctypes.c_int, [ctypes.POINTER(AttnArgs), ctypes.c_void_p]),
+    ('dkv_attend_workspace_bytes', ctypes.c_int64, [ctypes.c_void_p]),
+    ('dkv_attend', ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p]),
     ('dkv_attend_noalloc', ctypes.c_int, [ctypes.POINTER(AttnArgs), ctypes.c_void_p]),
     ('dkv_export', ctypes.c_int, [ctypes.POINTER(SegmentIO), ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32,
                                   ctypes.c_int32, ctypes.c_void_p]),
@@ -121,10 +140,11 @@ def lib_path():
 
 def load():
     """Loads libdkv.so once; raises if it has not been built."""
-    global _lib
+    global _lib, _zeroed_workspace
     if _lib is not None:
         return _lib
     path = lib_path()
+    _zeroed_workspace = 'inkernel' in os.path.basename(path)
     if not os.path.exists(path):
         raise RuntimeError(f'{path} is missing: build it first (python -c "import __graft_entry__ as g; g.build()")')
     lib = ctypes.CDLL(path)
@@ -136,6 +156,12 @@ def load():
         raise RuntimeError(f'libdkv ABI {lib.dkv_version()} != expected {ABI_VERSION}')
     _lib = lib
     return lib
+
+
+def workspace_uncleared():
+    """Whether dkv_attend takes a workspace of any bytes. (The in-kernel merge build, a measurement
+    build, wants zeroed arrival counters at its start.)"""
+    return not _zeroed_workspace
 
 
 def check(rc, what):
@@ -154,12 +180,17 @@ def stream_handle(device=None):
     """torch's current stream on `device` (a torch.device, an index or None: the current device) as
     a hipStream_t. Every launch asks: the current stream changes under torch.cuda.stream() and
     during graph capture."""
+    return ctypes.c_void_p(raw_stream(device))
+
+
+def raw_stream(device=None):
+    """stream_handle() as a plain address."""
     if _raw_stream is not None:
         if isinstance(device, str):
             device = torch.device(device)
         index = device.index if isinstance(device, torch.device) else device
-        return ctypes.c_void_p(_raw_stream(torch.cuda.current_device() if index is None else index))
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+        return _raw_stream(torch.cuda.current_device() if index is None else index)
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 def subblock_bytes(rows, bits):

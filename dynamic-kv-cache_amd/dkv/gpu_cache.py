@@ -30,6 +30,7 @@ BITS = (4, 8, 16)
 # does (src/gpu_kernels.py:93-94,102). 'fp32': fp32-accurate (split bf16 pairs on the MFMA path).
 PRECISIONS = {'bf16': 0, 'fp32': 1}
 PATHS = {'auto': 0, 'vector': 1, 'mfma': 2, 'short': 3}
+_ONE_SEGMENT = (0,) * (_lib.DKV_MAX_CHUNK_SEGS + 1)  # dkv_attn_args.seg_bounds of an unsegmented chunk
 SHORT_ROWS = 16  # query rows per KV head the short-chunk kernel takes (SHORT_ROWS of csrc/dkv_attn_common.h)
 
 
@@ -142,7 +143,8 @@ class GPUCache(_CacheBase):
         # Shared by forks, as the device table is.
         self.tiles_host = np.zeros(self.tiles.shape[0], dtype=TILE_DTYPE)
         self._tiles_host_ptr = self.tiles_host.ctypes.data  # fixed: the array is never replaced
-        self._workspace = None
+        self._tiles_host_bytes = self.tiles_host.view(np.uint8)
+        self._workspace = None  # split partials of the last call that needed any
         self._graph = None  # GraphSteps while launches read their step parameters from the device
         self._fused_args, self._fused_key = None, None  # the argument block _fused_attention() reuses
         for bits, n in planned:
@@ -165,13 +167,10 @@ class GPUCache(_CacheBase):
         seg = _Segment(start, n, bits, self.arena_used, tile0, frame)
         self.segments.append(seg)
         self.tile_starts.extend(range(start, start + n, TILE))
-        t = np.arange((n + TILE - 1) // TILE)
-        entries = self.tiles_host[tile0:tile0 + len(t)]
-        entries['offset'] = self.arena_used + t * slab_bytes(TILE, bits, self.layers, self.heads)
-        entries['token_start'] = start + t * TILE
-        entries['rows'] = np.minimum(n - t * TILE, TILE)
-        entries['bits'] = bits
-        entries['reserved'] = 0
+        slab = slab_bytes(TILE, bits, self.layers, self.heads)
+        for t in range((n + TILE - 1) // TILE):
+            _lib.TILE.pack_into(self._tiles_host_bytes, 16 * (tile0 + t), self.arena_used + t * slab,
+                                start + t * TILE, min(n - t * TILE, TILE), bits, 0)
         self.plan.append((start, start + n, bits, self.host_counts[bits]))
         self.host_counts[bits] += n
         self.arena_used += need
@@ -251,30 +250,39 @@ class GPUCache(_CacheBase):
 
     # -- hot path ----------------------------------------------------------
     @staticmethod
-    def _kv_view(x):
-        """[1, H, n, 64] view with contiguous rows, 16-byte aligned (copies otherwise)."""
-        if (x.stride(-1) != 1 or x.stride(1) % 8 or x.stride(2) % 8 or x.data_ptr() % 16
-                or x.dtype != torch.bfloat16):
+    def _rows(x):
+        """(view, address, strides) of a [1, H, n, 64] tensor as bf16 with contiguous rows, 16-byte
+        aligned (copies otherwise)."""
+        ptr, strides = x.data_ptr(), x.stride()
+        if strides[3] != 1 or strides[1] % 8 or strides[2] % 8 or ptr % 16 or x.dtype is not torch.bfloat16:
             x = x.to(torch.bfloat16).contiguous()
-        return x
+            ptr, strides = x.data_ptr(), x.stride()
+        return x, ptr, strides
+
+    @staticmethod
+    def _kv_view(x):
+        return GPUCache._rows(x)[0]
 
     def append(self, k, v, layer):
         """Packs the new tokens of one layer; returns the history length (src/gpu_cache.py:68-94)."""
-        if k.shape[0] != 1 or k.shape[-1] != self.dim or k.device.type != 'cuda':
+        shape = k.shape
+        if shape[0] != 1 or shape[-1] != self.dim or not k.is_cuda:
             raise ValueError('GPU cache requires CUDA, batch one and the configured head dimension')
-        if k.dim() != 4 or k.shape[1] != self.heads or v.shape != k.shape or v.device != k.device:
+        if len(shape) != 4 or shape[1] != self.heads or v.shape != shape or v.get_device() != k.get_device():
             raise ValueError(f'append expects k and v of shape [1, {self.heads}, n, {self.dim}]')
         if self._graph is not None:
             return self._graph.append(k, v, layer)
-        n = k.shape[-2]
+        n = shape[2]
         past, seg, write_tiles = self._claim(layer, n)
         if n:
-            k, v = self._kv_view(k), self._kv_view(v)
-            job = self._job(k, v, layer, past, n, seg, write_tiles)
-            lib = _lib.load()
-            _lib.check(lib.dkv_pack(ctypes.byref(job), self.arena.data_ptr(), self.arena_bytes,
-                                    self.tiles.data_ptr(), self.layers, self.heads,
-                                    _lib.stream_handle(self.device)), 'dkv_pack')
+            k, kp, ks = self._rows(k)
+            v, vp, vs = self._rows(v)
+            job = _lib.PACK_JOB.pack(kp, vp, ks[1], ks[2], vs[1], vs[2], seg.offset, seg.rows, seg.start,
+                                     past - seg.start, n, layer, seg.bits, seg.tile0, write_tiles)
+            rc = _lib.load().dkv_pack(job, self.arena.data_ptr(), self.arena_bytes, self.tiles.data_ptr(), self.layers,
+                                      self.heads, _lib.raw_stream(self.device))
+            if rc:
+                _lib.check(rc, 'dkv_pack')
         self.seen[layer] = past + n
         return past
 
@@ -459,10 +467,13 @@ class GPUCache(_CacheBase):
         return a
 
     def _workspace_for(self, nbytes):
-        # Split partials of the attention kernels: every call writes what its merge reads.
-        if self._workspace is None or self._workspace.numel() < nbytes or self._workspace.device != self.device:
-            self._workspace = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=self.device)
-        return self._workspace
+        # Split partials of the attention kernels: every call writes what its merge reads, so the bytes
+        # need no clearing. A block of its own for every call, from torch's allocator (stream-ordered
+        # reuse): calls on several streams or threads never share one. Clearing it cost a launch of its
+        # own, 2.4-4.6 us of GPU time beside the 8.6 us of a decode step's two kernels.
+        alloc = self.arena.new_empty if _lib.workspace_uncleared() else self.arena.new_zeros
+        self._workspace = ws = alloc(nbytes)
+        return ws
 
     def attend(self, q, k, v, layer, past, out_dtype=None, segments=None, path=0, splits=0, precision=None):
         """Causal attention of q over history [0, past) plus the native chunk (src/gpu_cache.py:96-104).
@@ -473,42 +484,66 @@ class GPUCache(_CacheBase):
         'mfma', 'short' (the short-chunk kernel, at most 16 query rows per KV head) or 'vector'; `precision` overrides the cache's 'bf16' / 'fp32'
         setting for this call.
         """
-        if precision is not None and precision not in PRECISIONS:
+        if precision is None:
+            precision = self.precision
+        elif precision not in PRECISIONS:
             raise ValueError(f'precision must be one of {sorted(PRECISIONS)}')
-        if isinstance(path, str) and path not in PATHS:
-            raise ValueError(f'path must be one of {sorted(PATHS)}')
-        n = q.shape[-2]
-        if q.dim() != 4 or q.shape[0] != 1 or q.shape[-1] != self.dim or q.shape[1] % self.heads:
+        if isinstance(path, str):
+            if path not in PATHS:
+                raise ValueError(f'path must be one of {sorted(PATHS)}')
+            path = PATHS[path]
+        shape, heads, d = q.shape, self.heads, self.dim
+        if len(shape) != 4 or shape[0] != 1 or shape[3] != d or shape[1] % heads:
             raise ValueError('attend expects q [1, q_heads, n, 64] with q_heads a multiple of heads')
-        if k.shape != (1, self.heads, n, self.dim) or v.shape != k.shape:
-            raise ValueError(f'attend expects the chunk k, v of shape [1, {self.heads}, {n}, {self.dim}]')
+        _, q_heads, n, _ = shape
+        if k.shape != (1, heads, n, d) or v.shape != k.shape:
+            raise ValueError(f'attend expects the chunk k, v of shape [1, {heads}, {n}, {d}]')
         if past + n > self.capacity or past > self.seen[layer]:
             raise ValueError('attend: history longer than the cache holds')
-        if q.device.type != 'cuda' or k.device != q.device or v.device != q.device:
+        index = q.get_device()
+        if not q.is_cuda or k.get_device() != index or v.get_device() != index:
             raise ValueError('attend requires CUDA tensors on one device')
         if segments is None:
             segments = self.chunk_segments
         if segments is not None and (segments[0] != 0 or segments[-1] != n):
             raise ValueError(f'chunk segments {segments} do not cover the {n}-token chunk')
-        if splits == 0 and q.shape[1] // self.heads * n > SHORT_ROWS:
+        if splits == 0 and q_heads // heads * n > SHORT_ROWS:
             splits = self.chunk_splits
         out_dtype = out_dtype or q.dtype
-        _check_dtype(out_dtype, 'attend output dtype')
-        q, k, v = self._kv_view(q), self._kv_view(k), self._kv_view(v)
-        out = torch.empty((1, n, q.shape[1], self.dim), dtype=out_dtype, device=q.device)
-        if self._graph is not None:
-            a = self._graph.attend_args(q, k, v, layer, out, segments, path, splits, precision)
-        else:
-            a = self.attend_args(q, k, v, layer, past, out, segments, path, splits, precision)
+        if out_dtype not in OUT_DTYPES:
+            _check_dtype(out_dtype, 'attend output dtype')
+        q, qp, qs = self._rows(q)
+        k, kp, ks = self._rows(k)
+        v, vp, vs = self._rows(v)
+        out = q.new_empty((1, n, q_heads, d), dtype=out_dtype)
         lib = _lib.load()
-        need = lib.dkv_attend_workspace_bytes(ctypes.byref(a))
-        if need:
-            # A captured graph keeps the workspace it recorded: graph launches use their
-            # GraphSteps' own buffer, so an ordinary call that grows the cache's buffer can never
-            # free memory a graph still writes.
-            ws = self._graph.workspace(need) if self._graph is not None else self._workspace_for(need)
-            a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
-        _lib.check(lib.dkv_attend(ctypes.byref(a), _lib.stream_handle(self.device)), 'dkv_attend')
+        if self._graph is not None or segments:
+            if self._graph is not None:
+                a = self._graph.attend_args(q, k, v, layer, out, segments, path, splits, precision)
+            else:
+                a = self.attend_args(q, k, v, layer, past, out, segments, path, splits, precision)
+            need = lib.dkv_attend_workspace_bytes(ctypes.byref(a))
+            if need:
+                # A captured graph keeps the workspace it recorded: graph launches use their
+                # GraphSteps' own buffer, never a block that is given back after the call.
+                ws = self._graph.workspace(need) if self._graph is not None else self._workspace_for(need)
+                a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+            rc = lib.dkv_attend(ctypes.byref(a), _lib.raw_stream(self.device))
+        else:
+            # attend_args() of one causal chunk as bytes (dkv_attn_args, field by field)
+            head = (qp, qs[1], qs[2], kp, ks[1], ks[2], vp, vs[1], vs[2], self.arena.data_ptr(), self.tiles.data_ptr(),
+                    self._tiles_before(past), past, layer, self.layers, heads, q_heads, n, 0, *_ONE_SEGMENT,
+                    d ** -0.5, out.data_ptr(), q_heads * d, d, out_dtype is torch.float32, int(path), splits,
+                    PRECISIONS[precision])
+            tail = (0, self._tiles_host_ptr)  # no step pair
+            a = _lib.ATTN_ARGS.pack(*head, 0, 0, *tail)
+            need = lib.dkv_attend_workspace_bytes(a)
+            if need:
+                ws = self._workspace_for(need)
+                a = _lib.ATTN_ARGS.pack(*head, ws.data_ptr(), need, *tail)
+            rc = lib.dkv_attend(a, _lib.raw_stream(self.device))
+        if rc:
+            _lib.check(rc, 'dkv_attend')
         return out
 
     def materialize(self, layer, out_dtype=None):
@@ -516,13 +551,13 @@ class GPUCache(_CacheBase):
         n = self.seen[layer]
         out_dtype = out_dtype or self.dtype
         _check_dtype(out_dtype, 'materialize output dtype')
-        out = torch.empty((2, self.heads, n, self.dim), dtype=out_dtype, device=self.device)
+        out = self.arena.new_empty((2, self.heads, n, self.dim), dtype=out_dtype)
         if n:
-            lib = _lib.load()
-            _lib.check(lib.dkv_reconstruct(self.arena.data_ptr(), self.tiles.data_ptr(), self._tiles_before(n), n,
-                                           layer, self.layers, self.heads, out.data_ptr(),
-                                           1 if out.dtype == torch.float32 else 0,
-                                           _lib.stream_handle(self.device)), 'dkv_reconstruct')
+            rc = _lib.load().dkv_reconstruct(self.arena.data_ptr(), self.tiles.data_ptr(), self._tiles_before(n), n,
+                                             layer, self.layers, self.heads, out.data_ptr(),
+                                             int(out_dtype is torch.float32), _lib.raw_stream(self.device))
+            if rc:
+                _lib.check(rc, 'dkv_reconstruct')
         return out[0:1], out[1:2]
 
     def update(self, key_states, value_states, layer_idx, cache_kwargs=None):
