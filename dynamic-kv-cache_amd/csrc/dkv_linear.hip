@@ -117,7 +117,9 @@ __global__ void __launch_bounds__(64 * WAVES) linear_kernel(const LinearArgs a) 
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     const int row = min((rg * RB + rb) * 16 + col, a.rows - 1);
-    xrow[rb] = x_tiled ? a.x + (int64_t)(rg * RB + rb) * a.kp * 1024 + 8 * lane : a.x + (int64_t)row * a.ldx + 8 * g;
+    // a tiled x ends with the block of its last row (the second block of a pair may be past it)
+    const int block = min(rg * RB + rb, (a.rows - 1) >> 4);
+    xrow[rb] = x_tiled ? a.x + (int64_t)block * a.kp * 1024 + 8 * lane : a.x + (int64_t)row * a.ldx + 8 * g;
   }
 
   constexpr int TILES = RB * NB, OUT = RB * NT;
@@ -315,6 +317,250 @@ __global__ void __launch_bounds__(64 * WAVES) linear_kernel(const LinearArgs a) 
   }
 }
 
+// The same projections for many rows (prompts, several frames at once), where linear_kernel reads
+// every weight tile again for each 16 or 32 rows. A workgroup of 4 waves (2 x 2) computes 64 x rows
+// by 64 weight rows. Per pair of MFMA steps (64 k) 64 + 64 rows go to LDS, 1 KB per 16 rows and step
+// in the order the lanes read them, so every LDS access is 1 KB of consecutive bytes.
+//
+// The arithmetic is linear_kernel's, operation for operation, so that a row's result does not
+// depend on how many rows its call has: that kernel's wave w accumulates the pairs w, w + 8, ... (a
+// chain) from zero, and the chains are added in wave order. Here a wave walks chain after chain.
+//
+// Loads go straight to LDS (global_load_lds), into one of TILE_RING buffers, TILE_RING - 1 pairs
+// ahead; one barrier per pair. (Through registers, the ds_writes took longer than the loads: gate/up
+// at 1000 rows 29.4 us, 17.8 with the writes left out.) What bounds it now is the rate at which a CU
+// takes bytes from L2, about 60 KB/us each however many CUs load: 245 KB per 64 x 64 tile of k 960.
+// The 960-wide decoder's projections, linear_kernel -> this (with the norm launch), us per launch:
+//   rows   Q/K/V            o_proj           gate/up          down_proj
+//    256   10.1 -> 11.1      6.4 ->  7.4     16.7 -> 12.6      8.1 -> 13.6
+//    512   16.4 -> 11.9     10.8 ->  7.6     26.5 -> 16.1     13.7 -> 13.9
+//   1000   29.4 -> 15.0     19.5 ->  8.2     50.6 -> 24.1     40.9 -> 14.5
+//   2048   60.4 -> 24.4     36.3 -> 14.1    103.6 -> 42.9     94.3 -> 21.5
+// Tiles of 128 x 64 and 128 x 128 (4 or 8 waves) were slower below 2048 rows (fewer workgroups, and
+// prologues and epilogues that nothing overlaps); a ring of 4 buffers changed nothing.
+constexpr int TILE_M = 64, TILE_N = 64, TILE_RING = 3;
+
+// A wave's operands of one MFMA step, out of LDS: two pieces from x and two from w on, the second 2 KB
+// after the first (the up piece of SiLU*up WSTEP bytes after the gate's). One asm block with its own
+// wait: as ordinary LDS loads they waited for every global_load_lds in flight at the head of the
+// pair loop.
+template <int WSTEP>
+__device__ __forceinline__ void lds_operands(uint32_t x, uint32_t w, Op8 (&xa)[2], Op8 (&wa)[2]) {
+  asm volatile(
+      "ds_read_b128 %0, %4\n ds_read_b128 %1, %4 offset:2048\n"
+      "ds_read_b128 %2, %5\n ds_read_b128 %3, %5 offset:%6\n s_waitcnt lgkmcnt(0)"
+      : "=&v"(xa[0].u), "=&v"(xa[1].u), "=&v"(wa[0].u), "=&v"(wa[1].u)
+      : "v"(x), "v"(w), "n"(WSTEP)
+      : "memory");
+}
+
+template <int EPI, int OPS>
+__global__ void __launch_bounds__(256, 3) linear_tile_kernel(const LinearArgs a) {
+  constexpr int NT = EPI == EPI_SILU_MUL ? TILE_N / 2 : TILE_N;  // output columns of the workgroup
+  constexpr int NH = EPI == EPI_SILU_MUL ? 1 : 2;                // 16-column blocks of them per wave
+  constexpr int XF = TILE_M / 8, F = XF + TILE_N / 8, FW = F / 4;  // 1 KB pieces of a pair: of x, in all, per wave
+  __shared__ __attribute__((aligned(1024))) u32x4 lds[TILE_RING * F][64];
+  const int b = blockIdx.x;
+  const int xcd = b & 7, j = b >> 3;
+  const int rg = j % a.row_groups;
+  const int ct = (j / a.row_groups) * 8 + xcd;
+  if (ct >= a.n_tiles) return;  // uniform over the workgroup
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int n0 = ct * NT, m0 = rg * TILE_M;
+  constexpr bool w_tiled = OPS & LAYOUT_W_TILED, x_tiled = OPS & LAYOUT_X_TILED;
+  const int last_block = (a.rows - 1) >> 4;
+
+  // Piece f of a pair: block f / 2 of x (then of w), MFMA step f % 2. A wave loads pieces wave,
+  // wave + 4, ...
+  const uint16_t* src[FW];
+#pragma unroll
+  for (int q = 0; q < FW; ++q) {
+    const int f = wave + 4 * q, h = f & 1;
+    if (4 * q < XF) {  // rows past the end read the last row (block) and are not stored
+      const int row = m0 + 16 * (f >> 1);
+      src[q] = x_tiled ? a.x + (int64_t)min(row >> 4, last_block) * a.kp * 1024 + 512 * h + 8 * lane
+                       : a.x + (int64_t)min(row + col, a.rows - 1) * a.ldx + 32 * h + 8 * g;
+    } else {
+      const int cb = (f - XF) >> 1;
+      const int r = EPI == EPI_SILU_MUL && cb >= NT / 16 ? a.up + n0 + 16 * (cb - NT / 16) : n0 + 16 * cb;
+      src[q] = w_tiled ? a.w + (int64_t)(r >> 4) * a.kp * 1024 + 512 * h + 8 * lane
+                       : a.w + (int64_t)(r + col) * a.ldw + 32 * h + 8 * g;
+    }
+  }
+  auto next = [&](int p) {  // the pair after p: the next of its chain, or the next chain's first
+    const int q = p + 8;
+    return q < a.kp ? q : (p & 7) + 1;
+  };
+  // Past the last pair the last one is loaded again (never used), so that every pair has FW loads
+  // after it.
+  int pl = 0, loaded = 0;  // pair loaded next and its place in the order
+  int fill = 0;  // the buffer loaded next
+  auto load_next = [&]() {
+#pragma unroll
+    for (int q = 0; q < FW; ++q) {
+      const uint16_t* from = src[q] + ((4 * q < XF ? x_tiled : w_tiled) ? 1024 * pl : 64 * pl);
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)from,
+                                       (__attribute__((address_space(3))) void*)lds[fill * F + wave + 4 * q], 16, 0, 0);
+    }
+    fill = fill + 1 == TILE_RING ? 0 : fill + 1;
+    if (++loaded < a.kp) pl = next(pl);
+  };
+
+  f32x4_t acc[2][2], sum[2][2];  // the chain in progress; the chains done
+#pragma unroll
+  for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) {
+      acc[mb][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      sum[mb][nb] = f32x4_t{-0.f, -0.f, -0.f, -0.f};  // -0 + x is x, for every x
+    }
+  // LDS byte addresses of this wave's first x and w piece in buffer 0
+  const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + 16 * lane;
+  const uint32_t xl = base + 4096 * wm, wl = base + 1024 * XF + 2048 * wn * NH;
+  constexpr int WSTEP = EPI == EPI_SILU_MUL ? 2048 * (NT / 16) : 2048;
+  auto compute = [&](uint32_t at) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      Op8 xa[2], wa[2];
+      lds_operands<WSTEP>(xl + at + 1024 * h, wl + at + 1024 * h, xa, wa);
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb)
+          acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[nb].v, xa[mb].v, acc[mb][nb], 0, 0, 0);
+    }
+  };
+#pragma unroll
+  for (int k = 0; k < TILE_RING - 1; ++k) load_next();
+  int p = 0;        // pair being computed
+  uint32_t at = 0;  // its buffer, in bytes
+  for (int s = 0; s < a.kp; ++s) {
+    // The pair's pieces have landed (this wave's: at most the loads of the TILE_RING - 2 pairs after it
+    // are under way; the other waves': the barrier), and every wave is past the pair before it,
+    // whose buffer the next loads overwrite.
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((TILE_RING - 2) * FW) : "memory");
+    __builtin_amdgcn_s_barrier();
+    load_next();
+    compute(at);
+    at = at + 1024 * F == 1024 * F * TILE_RING ? 0 : at + 1024 * F;
+    if (p + 8 >= a.kp) {  // the chain's last pair
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            sum[mb][nb][e] += acc[mb][nb][e];
+            acc[mb][nb][e] = 0.f;
+          }
+    }
+    p = next(p);
+  }
+
+  // The loads past the last pair still write this workgroup's LDS.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+  uint2 resv[2][2];
+  if constexpr (EPI == EPI_RESIDUAL) {
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb) {
+        const int row = min(m0 + 16 * (wm * 2 + mb) + col, a.rows - 1), c = n0 + 16 * (wn * 2 + nb) + 4 * g;
+        resv[mb][nb] = *reinterpret_cast<const uint2*>(
+            a.res + ((a.layout & LAYOUT_RES_TILED) ? tiled_offset(row, c, a.up >> 6) : (int64_t)row * a.ldr + c));
+      }
+  }
+#pragma unroll
+  for (int mb = 0; mb < 2; ++mb) {
+    const int row = m0 + 16 * (wm * 2 + mb) + col;
+    if (row >= a.rows) continue;
+#pragma unroll
+    for (int nb = 0; nb < NH; ++nb) {
+      const int c = n0 + 16 * (wn * NH + nb) + 4 * g;
+      float y[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = round_bf16(sum[mb][nb][e]);
+      if constexpr (EPI == EPI_RESIDUAL) {
+        const uint2 r = resv[mb][nb];
+        y[0] += bf16_lo(r.x);
+        y[1] += bf16_hi(r.x);
+        y[2] += bf16_lo(r.y);
+        y[3] += bf16_hi(r.y);
+      } else if constexpr (EPI == EPI_SILU_MUL) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          y[e] = round_bf16(y[e] / (1.f + expf(-y[e]))) * round_bf16(sum[mb][NH + nb][e]);
+      }
+      uint16_t* dst = a.out + ((a.layout & LAYOUT_OUT_TILED) ? tiled_offset(row, c, a.up >> 6) : (int64_t)row * a.ldo + c);
+      *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3]));
+    }
+  }
+}
+
+// RMSNorm of x rows into the MFMA-tiled layout, for linear_tile_kernel: linear_kernel's prologue as
+// a launch of its own (there every workgroup normalizes its x rows again; with 16 times the rows per
+// weight tile that work is worth doing once). One workgroup per 16 rows; wave w sums and normalizes
+// pairs w, w + 8, ..., in linear_kernel's order.
+template <int CH, bool XT>
+__global__ void __launch_bounds__(512)
+rms_tiled_kernel(const uint16_t* __restrict__ x, int64_t ldx, const uint16_t* __restrict__ norm,
+                 uint16_t* __restrict__ out, int rows, int k, int kp, float eps) {
+  constexpr int WAVES = 8;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
+  const int64_t tile = (int64_t)blockIdx.x * kp * 1024 + 8 * lane;
+  const uint16_t* xr = XT ? x + tile : x + (int64_t)min((int)blockIdx.x * 16 + col, rows - 1) * ldx + 8 * g;
+  Op8 xa[CH][2], gn[CH][2];
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+    const int p = min(wave + WAVES * i, kp - 1);  // a pair past kp is loaded and skipped
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      xa[i][h].u = *reinterpret_cast<const u32x4*>(xr + (XT ? 1024 * p + 512 * h : 64 * p + 32 * h));
+      gn[i][h].u = *reinterpret_cast<const u32x4*>(norm + 64 * p + 32 * h + 8 * g);
+    }
+  }
+  __shared__ float ssum[WAVES][16];
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+    if (wave + WAVES * i < kp)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float lo = bf16_lo(xa[i][h].u[e]), hi = bf16_hi(xa[i][h].u[e]);
+          ss = __fmaf_rn(lo, lo, ss);
+          ss = __fmaf_rn(hi, hi, ss);
+        }
+  }
+  ss = lane_group_sum(ss);
+  if (g == 0) ssum[wave][col] = ss;
+  __syncthreads();
+  float tot = 0.f;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) tot += ssum[w][col];
+  const float rstd = 1.f / sqrtf(tot / (float)k + eps);
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+    const int p = wave + WAVES * i;
+    if (p >= kp) continue;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      u32x4 y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t xv = xa[i][h].u[e], gv = gn[i][h].u[e];
+        y[e] = pack_bf16(round_bf16(bf16_lo(xv) * rstd) * bf16_lo(gv), round_bf16(bf16_hi(xv) * rstd) * bf16_hi(gv));
+      }
+      *reinterpret_cast<u32x4*>(out + tile + 1024 * p + 512 * h) = y;  // padding rows repeat the last row
+    }
+  }
+}
+
 bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 // Launch shapes, from graph-replay timings of the 960-wide decoder's projections at 64 rows
@@ -325,15 +571,18 @@ bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 // the second read of each weight tile they bring (64 rows per workgroup: 13.3 us, 32: 11.4 us).
 struct Shape {
   int ch, nt, waves, rb;
+  bool tile;  // linear_tile_kernel
 };
 
 constexpr int MAX_CH = 5;       // pairs per wave: k <= 5 * 8 * 64 = 2560
 constexpr int MAX_NORM_CH = 2;  // with the RMSNorm prologue (k <= 1024), which keeps those
                                 // variants out of scratch
 
-Shape pick(int n_out, int kp, int epilogue) {
+Shape pick(int rows, int n_out, int kp, bool norm, int epilogue) {
   Shape s;
   s.waves = 8;
+  s.ch = (kp + s.waves - 1) / s.waves;  // every pair of a wave in registers at once
+  s.tile = false;
   if (epilogue == EPI_SILU_MUL) {  // 32 gate and 32 up weight rows, 32 x rows
     s.nt = 2;
     s.rb = 2;
@@ -341,7 +590,20 @@ Shape pick(int n_out, int kp, int epilogue) {
     s.nt = (n_out % 32 == 0 && n_out / 16 > 64) ? 2 : 1;
     s.rb = 1;
   }
-  s.ch = (kp + s.waves - 1) / s.waves;  // every pair of a wave in registers at once
+  // Many rows: linear_tile_kernel, from the number of linear_kernel workgroups on at which it was
+  // faster (table above; 256 CUs). SiLU*up: as soon as they are more than one per CU (rows 96 -> 128:
+  // 7.2 -> 11.9 us, tiles 10.7 with the norm launch). Other projections: k 960 at 1000 to 1200
+  // workgroups (o_proj 256 rows 6.4 against 7.4 us, 384 rows 8.6 against 7.5; Q/K/V 256 rows 10.1
+  // against 11.1, 384 rows 13.9 against 11.5), k 2560 at 1920 (512 rows 13.7 against 13.9, 768 rows
+  // 20.7 against 14.3).
+  const int cols = 16 * s.nt, per = epilogue == EPI_SILU_MUL ? 2 : 1;
+  const int64_t groups = (int64_t)((rows + 16 * s.rb - 1) / (16 * s.rb)) * (n_out / cols);
+  const int64_t most = epilogue == EPI_SILU_MUL ? 256 : (kp > 16 ? 2000 : 1100);
+  if (!norm && n_out * per % TILE_N == 0 && groups > most) {
+    s.tile = true;
+    s.nt = TILE_N / per / 16;
+    s.rb = TILE_M / 16;
+  }
   return s;
 }
 
@@ -350,6 +612,12 @@ void launch_one(const LinearArgs& a, hipStream_t st) {
   const int groups = (a.n_tiles + 7) / 8;
   const unsigned blocks = (unsigned)groups * 8u * (unsigned)a.row_groups;
   hipLaunchKernelGGL((linear_kernel<CH, NT, WAVES, RB, EPI, NORM, OPS>), dim3(blocks), dim3(64 * WAVES), 0, st, a);
+}
+
+template <int EPI, int OPS>
+void launch_tile(const LinearArgs& a, hipStream_t st) {
+  const unsigned blocks = (unsigned)((a.n_tiles + 7) / 8) * 8u * (unsigned)a.row_groups;
+  hipLaunchKernelGGL((linear_tile_kernel<EPI, OPS>), dim3(blocks), dim3(256), 0, st, a);
 }
 
 template <int NT, int WAVES, int RB, int EPI, bool NORM, int OPS>
@@ -372,6 +640,8 @@ void launch_ch(int ch, const LinearArgs& a, hipStream_t st) {
 
 template <int EPI, bool NORM, int OPS>
 void launch_ops(const Shape& s, const LinearArgs& a, hipStream_t st) {
+  if constexpr (!NORM)
+    if (s.tile) return launch_tile<EPI, OPS>(a, st);
   if constexpr (EPI == EPI_SILU_MUL) {
     launch_ch<2, 8, 2, EPI, NORM, OPS>(s.ch, a, st);
   } else {
@@ -402,10 +672,10 @@ int dkv_linear_supported(int32_t rows, int32_t n, int32_t k, int32_t has_norm, i
   const int n_out = epilogue == EPI_SILU_MUL ? n / 2 : n;
   if (epilogue == EPI_SILU_MUL && (n & 1)) return 0;
   if (n_out % 16) return 0;
-  const Shape s = pick(n_out, k / 64, epilogue);
+  const Shape s = pick(rows, n_out, k / 64, has_norm, epilogue);
   const int max_ch = has_norm ? MAX_NORM_CH : (epilogue == EPI_SILU_MUL ? 4 : MAX_CH);  // register budget
   if (s.ch > max_ch) return 0;
-  if (s.nt == 2 && n_out % 32) return 0;
+  if (n_out % (16 * s.nt)) return 0;
   return 1;
 }
 
@@ -431,7 +701,7 @@ int dkv_linear_tiled(const void* x, int64_t x_row_stride, const void* w, int64_t
     return DKV_EINVAL;
   }
   if (rows == 0) return 0;
-  const Shape s = pick(n_out, k / 64, epilogue);
+  const Shape s = pick(rows, n_out, k / 64, norm, epilogue);
   LinearArgs a;
   a.x = static_cast<const uint16_t*>(x);
   a.ldx = x_row_stride;
@@ -455,6 +725,38 @@ int dkv_linear_tiled(const void* x, int64_t x_row_stride, const void* w, int64_t
   else if (epilogue == EPI_RESIDUAL)
     norm ? launch_epi<EPI_RESIDUAL, true>(s, a, st) : launch_epi<EPI_RESIDUAL, false>(s, a, st);
   else norm ? launch_epi<EPI_SILU_MUL, true>(s, a, st) : launch_epi<EPI_SILU_MUL, false>(s, a, st);
+  return (int)hipGetLastError();
+}
+
+int dkv_linear_prenorm(int32_t rows, int32_t n, int32_t k, int32_t epilogue) {
+  if (!dkv_linear_supported(rows, n, k, 1, epilogue) || !dkv_linear_supported(rows, n, k, 0, epilogue)) return 0;
+  return pick(rows, epilogue == EPI_SILU_MUL ? n / 2 : n, k / 64, false, epilogue).tile;
+}
+
+int dkv_rms_norm_tiled(const void* x, int64_t x_row_stride, const void* weight, void* out, int32_t rows, int32_t k,
+                       float eps, int32_t layout, void* stream) {
+  clear_error();
+  const bool xt = layout & LAYOUT_X_TILED;
+  if (!x || !weight || !out || rows < 0 || k <= 0 || (k & 63) || k > 64 * 8 * MAX_NORM_CH || !al16(x) || !al16(weight) ||
+      !al16(out) || (layout & ~LAYOUT_X_TILED) || (!xt && ((x_row_stride & 7) || x_row_stride < k))) {
+    set_error("dkv_rms_norm_tiled: bad arguments (rows %d, k %d, layout %d; k a multiple of 64, at most %d, 16-byte "
+              "aligned bf16 rows)", rows, k, layout, 64 * 8 * MAX_NORM_CH);
+    return DKV_EINVAL;
+  }
+  if (rows == 0) return 0;
+  const dim3 grid((rows + 15) / 16);
+  const auto* xp = static_cast<const uint16_t*>(x);
+  const auto* wp = static_cast<const uint16_t*>(weight);
+  auto* op = static_cast<uint16_t*>(out);
+  hipStream_t st = (hipStream_t)stream;
+  const int kp = k / 64;
+  if (kp <= 8) {
+    if (xt) hipLaunchKernelGGL((rms_tiled_kernel<1, true>), grid, dim3(512), 0, st, xp, x_row_stride, wp, op, rows, k, kp, eps);
+    else hipLaunchKernelGGL((rms_tiled_kernel<1, false>), grid, dim3(512), 0, st, xp, x_row_stride, wp, op, rows, k, kp, eps);
+  } else {
+    if (xt) hipLaunchKernelGGL((rms_tiled_kernel<2, true>), grid, dim3(512), 0, st, xp, x_row_stride, wp, op, rows, k, kp, eps);
+    else hipLaunchKernelGGL((rms_tiled_kernel<2, false>), grid, dim3(512), 0, st, xp, x_row_stride, wp, op, rows, k, kp, eps);
+  }
   return (int)hipGetLastError();
 }
 

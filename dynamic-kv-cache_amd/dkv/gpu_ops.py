@@ -104,6 +104,11 @@ def _linear_supported(rows, n, k, norm, epilogue):
     return bool(_lib.load().dkv_linear_supported(rows, n, k, norm, epilogue))
 
 
+@functools.lru_cache(maxsize=None)
+def _prenorm(rows, n, k, epilogue):
+    return bool(_lib.load().dkv_linear_prenorm(rows, n, k, epilogue))
+
+
 def linear_covered(rows, weight, norm=False, epilogue=LINEAR_PLAIN):
     """Whether dkv_linear has a launch for x [rows, weight.shape[1]] . weight^T with this prologue/epilogue."""
     return _weight_rows(weight) and _linear_supported(rows, weight.shape[0], weight.shape[1], int(norm), epilogue)
@@ -187,6 +192,13 @@ def linear(x, weight, norm=None, eps=1e-6, residual=None, silu_mul=False, weight
         return None
     out = torch.empty(((rows + 15) // 16 * 16 if out_tiled else rows, n_out), dtype=x.dtype, device=x.device)
     w = weight if weight_tiled is None else weight_tiled
+    if norm is not None and _prenorm(rows, weight.shape[0], k, epi):  # many rows: normalized once, in a launch of its own
+        xn = x.new_empty(((rows + 15) // 16 * 16, k))
+        _lib.check(_lib.load().dkv_rms_norm_tiled(x2.data_ptr(), x2.stride(0), norm.data_ptr(), xn.data_ptr(), rows, k,
+                                                  float(eps), layout & LINEAR_X_TILED, _lib.stream_handle(x.device)),
+                   'dkv_rms_norm_tiled')
+        x2, norm = xn, None
+        layout |= LINEAR_X_TILED
     _lib.check(_lib.load().dkv_linear_tiled(
         x2.data_ptr(), x2.stride(0), w.data_ptr(), w.stride(0), rows, weight.shape[0], k,
         None if norm is None else norm.data_ptr(), float(eps), epi, None if r2 is None else r2.data_ptr(),
@@ -204,7 +216,8 @@ class _LayerPlan:
     module swaps a parameter's storage in place), their row strides and row counts, the norm
     epsilons and the head counts."""
     __slots__ = ('qkv_w', 'o_w', 'gu_w', 'd_w', 'ln1_w', 'ln2_w', 'qkv_args', 'o_args', 'gu_args', 'd_args',
-                 'eps1', 'eps2', 'q_heads', 'kv_heads', 'eager_ok', 'layer_idx', 'width', 'inter')
+                 'eps1', 'eps2', 'q_heads', 'kv_heads', 'eager_ok', 'layer_idx', 'width', 'inter', 'norm1_apart',
+                 'norm2_apart')
 
     def holds(self, layer):
         # the modules' own dicts: nn.Module attribute lookups cost more than the rest of this check
@@ -284,6 +297,9 @@ def _layer_plan(layer, n, width):
     # the eager launches split q | k | v as dkv_rope_pack does: 64-wide heads, K and V alike
     p.eager_ok = hd == 64 and sizes[1] == sizes[2] and p.qkv_w.shape[0] == sum(sizes) and sizes[0] % hd == 0
     p.layer_idx, p.width, p.inter = attn.layer_idx, width, p.gu_w.shape[0] // 2
+    # many rows: the norms as launches of their own, before Q/K/V and gate/up
+    p.norm1_apart = _prenorm(n, p.qkv_w.shape[0], width, LINEAR_PLAIN)
+    p.norm2_apart = _prenorm(n, p.gu_w.shape[0], width, LINEAR_SILU_MUL)
     plans[(n, width)] = p
     return p
 
@@ -314,23 +330,35 @@ def _fused_layer_eager(p, tiles, h, n, cache, cos, sin):
             gl |= LINEAR_X_TILED
             dl |= LINEAR_RES_TILED
     # element offsets of [qkv | q,k,v | attention out | h2 | act], each n rows (multiples of 64
-    # columns; act in rows rounded up to 16 when tiled)
+    # columns; h2 and act in rows rounded up to 16 when tiled)
     o_qkvo = n * qrows
     o_att = o_qkvo + n * qrows
     o_h2 = o_att + n * ok
     n16 = (n + 15) // 16 * 16
     o_act = o_h2 + n16 * orows
-    scratch = torch.empty(o_act + n16 * inter, dtype=torch.bfloat16, device=h.device)
+    o_norm = o_act + n16 * inter  # the normalized rows, tiled, where a norm is a launch of its own
+    apart = p.norm1_apart or p.norm2_apart
+    scratch = torch.empty(o_norm + (n16 * width if apart else 0), dtype=torch.bfloat16, device=h.device)
     out = torch.empty((1, n, drows), dtype=torch.bfloat16, device=h.device)
     base = scratch.data_ptr()
     xp, qkv, att, h2, act = h.data_ptr(), base, base + 2 * o_att, base + 2 * o_h2, base + 2 * o_act
-    _lib.check(lib.dkv_linear_tiled(xp, width, qw.data_ptr(), qld, n, qrows, qk, p.ln1_w.data_ptr(), p.eps1,
+    xn = base + 2 * o_norm
+    qx, norm1 = xp, p.ln1_w.data_ptr()
+    if p.norm1_apart:
+        _lib.check(lib.dkv_rms_norm_tiled(xp, width, norm1, xn, n, width, p.eps1, 0, stream), 'dkv_rms_norm_tiled')
+        qx, norm1, ql = xn, None, ql | LINEAR_X_TILED
+    _lib.check(lib.dkv_linear_tiled(qx, width, qw.data_ptr(), qld, n, qrows, qk, norm1, p.eps1,
                                     LINEAR_PLAIN, None, 0, qkv, qrows, ql, stream), 'dkv_linear')
     cache._fused_attention(n, p.q_heads, p.layer_idx, qkv, qrows, cos.data_ptr(), sin.data_ptr(), cos.stride(0),
                            base + 2 * o_qkvo, att, stream)
     _lib.check(lib.dkv_linear_tiled(att, ok, ow.data_ptr(), old, n, orows, ok, None, 1e-6, LINEAR_RESIDUAL, xp,
                                     width, h2, orows, ol, stream), 'dkv_linear')
-    _lib.check(lib.dkv_linear_tiled(h2, width, gw.data_ptr(), gld, n, grows, gk, p.ln2_w.data_ptr(), p.eps2,
+    gx, norm2 = h2, p.ln2_w.data_ptr()
+    if p.norm2_apart:
+        _lib.check(lib.dkv_rms_norm_tiled(h2, width, norm2, xn, n, width, p.eps2, gl & LINEAR_X_TILED, stream),
+                   'dkv_rms_norm_tiled')
+        gx, norm2, gl = xn, None, gl | LINEAR_X_TILED
+    _lib.check(lib.dkv_linear_tiled(gx, width, gw.data_ptr(), gld, n, grows, gk, norm2, p.eps2,
                                     LINEAR_SILU_MUL, None, 0, act, inter, gl, stream), 'dkv_linear')
     _lib.check(lib.dkv_linear_tiled(act, inter, dw.data_ptr(), dld, n, drows, dk, None, 1e-6, LINEAR_RESIDUAL, h2,
                                     width, out.data_ptr(), drows, dl, stream), 'dkv_linear')

@@ -330,6 +330,18 @@ int dkv_linear_tiled(const void* x, int64_t x_row_stride, const void* w, int64_t
                      int32_t epilogue, const void* residual, int64_t residual_row_stride,
                      void* out, int64_t out_row_stride, int32_t layout, void* stream);
 
+/* RMSNorm of x rows [rows, k] (k a multiple of 64, at most 1024) into the
+ * MFMA-tiled layout [rows rounded up to 16, k]: what dkv_linear's prologue forms,
+ * bit for bit, as a launch of its own, whose out is the x of dkv_linear_tiled
+ * calls with DKV_LINEAR_X_TILED (padding rows repeat the last row). layout: 0 or
+ * DKV_LINEAR_X_TILED (x tiled). dkv_linear_prenorm says whether a projection with
+ * a norm is faster that way (1) or with dkv_linear's norm_weight (0): from some
+ * hundred rows on. No counterpart in the reference (src/gpu_ops.py:9-12 is its
+ * norm). */
+int dkv_rms_norm_tiled(const void* x, int64_t x_row_stride, const void* weight, void* out, int32_t rows,
+                       int32_t k, float eps, int32_t layout, void* stream);
+int dkv_linear_prenorm(int32_t rows, int32_t n, int32_t k, int32_t epilogue);
+
 #ifdef __cplusplus
 }
 #endif
