@@ -15,6 +15,7 @@
 // value, well under the bf16 output's rounding, at half the partial traffic).
 // Softmax runs in base 2: x = score * scale * log2(e).
 #include "dkv_attn_common.h"
+#include "dkv_attn_prompt.h"
 #include "dkv_merge.h"
 #include <mutex>
 
@@ -504,6 +505,21 @@ static Plan make_plan(const dkv_attn_args& a) {
   return p;
 }
 
+// Calls that take the long-chunk kernels (dkv_attn_prompt.hip): default plans (graph replays, explicit
+// split counts and paths keep the frame-chunk kernel) with PROMPT_FROM query rows over all Q heads and
+// a full workgroup of them per KV head. Their third launch and their unpacked keys cost about 8 us,
+// which the frame-chunk kernel's idle CUs, masked units and repeated dequantization pass from there
+// on; frame-chunk -> long-chunk kernels, us per call, bf16 (q_heads x nq rows):
+//   15 / 5 heads  3840 rows (256 past 1024) 16.4 -> 17.1   4800 (320 past 1024) 18.8 -> 17.3
+//   32 / 8 heads  3200 rows (100 past  500) 13.8 -> 15.2   6400 (200 past 1000) 22.0 -> 18.4
+//   16 / 8 heads  4096 rows (256 past 1024) 16.5 -> 17.3   8192 (512 past 1024) 24.0 -> 18.4
+//    9 / 3 heads  2880 rows (320 past 1024) 15.1 -> 16.2   4608 (512 past 1024) 18.1 -> 16.8
+static constexpr int64_t PROMPT_FROM = 4500;
+static bool prompt_route(const dkv_attn_args& a) {
+  return a.path == 0 && a.splits <= 0 && !a.step && (int64_t)a.q_heads * a.nq >= PROMPT_FROM &&
+         (int64_t)(a.q_heads / a.heads) * a.nq >= PROMPT_ROWS;
+}
+
 // Workspace bytes of a plan: the split partials (none for one split), after the arrival counters in
 // the in-kernel merge build.
 static int64_t workspace_bytes(const Plan& p) {
@@ -609,7 +625,7 @@ extern "C" {
 int64_t dkv_attend_workspace_bytes(const dkv_attn_args* args) {
   if (!args || args->heads <= 0 || args->q_heads <= 0 || args->q_heads % args->heads || args->nq <= 0)
     return 0;
-  return workspace_bytes(make_plan(*args));
+  return prompt_route(*args) ? prompt_plan(*args, num_cus()).bytes() : workspace_bytes(make_plan(*args));
 }
 
 int dkv_attend(const dkv_attn_args* args, void* stream) {
@@ -620,13 +636,18 @@ int dkv_attend(const dkv_attn_args* args, void* stream) {
   }
   const dkv_attn_args& a = *args;
   if (int rc = check_args(a)) return rc;
-  const Plan p = make_plan(a);
-  const int64_t need = workspace_bytes(p);
+  const bool prompt = prompt_route(a);
+  PromptPlan pp;
+  Plan p;
+  if (prompt) pp = prompt_plan(a, num_cus());
+  else p = make_plan(a);
+  const int64_t need = prompt ? pp.bytes() : workspace_bytes(p);
   if (need > 0 && (!a.workspace || a.workspace_bytes < need)) {
     set_error("dkv_attend: workspace of %lld bytes needed, %lld given", (long long)need,
               (long long)a.workspace_bytes);
     return DKV_EINVAL;
   }
+  if (prompt) return launch_attn_prompt(a, pp, a.workspace, (hipStream_t)stream);
   return launch_attend(a, p, a.workspace, (hipStream_t)stream);
 }
 
@@ -638,6 +659,15 @@ int dkv_attend_noalloc(const dkv_attn_args* args, void* stream) {
   }
   const dkv_attn_args& a = *args;
   if (int rc = check_args(a)) return rc;
+  if (prompt_route(a)) {
+    // (a chunk whose unpacked keys and partials pass the scratch buffer runs the frame-chunk plan)
+    const PromptPlan pp = prompt_plan(a, num_cus());
+    if (pp.bytes() <= DKV_NOALLOC_SCRATCH_BYTES) {
+      void* ws = nullptr;
+      if (int rc = scratch_address(&ws)) return rc;
+      return launch_attn_prompt(a, pp, ws, (hipStream_t)stream);
+    }
+  }
   const Plan p = make_plan(a);
   const int64_t need = workspace_bytes(p);
   if (need > DKV_NOALLOC_SCRATCH_BYTES) {

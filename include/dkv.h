@@ -89,8 +89,8 @@ typedef struct dkv_attn_args {
   void* out;             /* [nq, q_heads, 64] with the strides below */
   int64_t out_tok_stride, out_head_stride;
   int32_t out_dtype;     /* 0 = bf16, 1 = fp32 */
-  int32_t path;          /* 0 = auto (the MFMA frame-chunk kernel, the fastest measured for every
-                            chunk length, decode steps included),
+  int32_t path;          /* 0 = auto (the MFMA frame-chunk kernel, decode steps included; the
+                            long-chunk kernels for prompts of several hundred tokens),
                             1 = vector, 2 = MFMA (frame chunks), 3 = short chunk (decode steps) */
   int32_t splits;        /* 0 = auto; history split count per KV head */
   int32_t precision;     /* 0 = the reference kernel's bf16 rounding of K, V and p
@@ -183,12 +183,16 @@ int dkv_reconstruct(const void* arena, const dkv_tile* tiles, int32_t n_tiles,
                     int32_t n_tokens, int32_t layer, int32_t layers, int32_t heads,
                     void* out, int32_t out_dtype, void* stream);
 
-/* Workspace bytes dkv_attend needs for these arguments. */
+/* Workspace bytes dkv_attend needs for these arguments: the split partials, and for a long chunk
+ * (path 0) its keys unpacked, heads * (past + nq) * 256 bytes (512 at precision 1). */
 int64_t dkv_attend_workspace_bytes(const dkv_attn_args* args);
 
 /* Fused packed-history causal GQA attention. Replaces GPUCache.attend's
  * packed_attention launch (src/gpu_cache.py:96-104, src/gpu_kernels.py:71-105).
- * Every chunk length runs a split-history MFMA kernel by default (path 0/2);
+ * Frames, candidate batches and decode steps run a split-history MFMA kernel
+ * (path 0/2); long chunks (path 0, 4500 query rows or more over all Q heads, no
+ * step pair and no explicit split count) unpack the keys once and run a causal
+ * MFMA kernel over ranges of them (three launches);
  * path 3 runs short chunks (at most 16 query rows per KV head, e.g. decode
  * steps) on a kernel with two waves per 64-key tile. A merge kernel combines
  * the history splits of either in a second launch.
@@ -206,7 +210,9 @@ int dkv_attend(const dkv_attn_args* args, void* stream);
  * args->workspace and args->workspace_bytes are ignored. Results equal
  * dkv_attend's for the same arguments. A call whose partials need more than
  * DKV_NOALLOC_SCRATCH_BYTES (dkv_attend_workspace_bytes) returns DKV_EINVAL
- * without launching; the metric's shapes need at most 13 MB. The first call on
+ * without launching; the metric's shapes need at most 13 MB. A long chunk whose
+ * unpacked keys do not fit runs the frame-chunk kernel instead (equal within the
+ * rounding of its precision), and is refused only if that needs more as well. The first call on
  * a device looks the buffer's address up (hipGetSymbolAddress): make that call
  * before capturing a graph. Calls share their device's buffer, so two calls on
  * one device that may overlap in time (different streams) race; serialize them

@@ -101,3 +101,103 @@ def test_tiled_x_ends_with_its_last_block(cuda):
     buf[:16] = gpu_ops.mfma_tiled(x)
     got = gpu_ops.linear(buf[:16], w, silu_mul=True, x_tiled=True, rows=9)
     assert torch.equal(got, gpu_ops.linear(x, w, silu_mul=True))
+
+
+def _dense(c, case, past, starts, dtype):
+    """(output, attention over |v|) [nq, Hq, 64] in float64 from the cache's own dequantized history,
+    K and V rounded to `dtype` as the kernel's precision does."""
+    k, v = (x[0, :, :past].double() for x in c.materialize(0, dtype))
+    q, kn, vn = (case[x].to(k.device).double() for x in ('q', 'k_new', 'v_new'))
+    k, v = torch.cat((k, kn), 1), torch.cat((v, vn), 1)
+    n, group = q.shape[1], q.shape[0] // k.shape[0]
+    rows = torch.arange(n, device=k.device)
+    mask = torch.ones(n, past + n, dtype=torch.bool, device=k.device)
+    mask[:, past:] = (rows[None] <= rows[:, None]) & (rows[None] >= starts.to(k.device)[:, None])
+    out, mag = (torch.empty(n, q.shape[0], 64, dtype=torch.float64, device=k.device) for _ in range(2))
+    for h in range(q.shape[0]):
+        p = (q[h] @ k[h // group].t().contiguous() / 8).masked_fill_(~mask, float('-inf')).softmax(-1)
+        out[:, h], mag[:, h] = p @ v[h // group], p @ v[h // group].abs()
+    return out, mag
+
+
+@pytest.mark.parametrize('heads,group,nq,past,tiles', [
+    (5, 3, 300, 0, 'none'),         # no history; the first row sees one key
+    (5, 3, 301, 1, 'frames'),       # one key of history, an odd chunk
+    (5, 3, 608, 999, 'frames'),     # past not a multiple of 64
+    (8, 4, 256, 4096, 'frames'),    # the history ends on a unit
+    (8, 2, 282, 700, 'ones'),       # one-token tiles (decode steps), 700 of them: past the table window
+    (1, 1, 4500, 77, 'frames'),     # one head; the last group of rows is partly empty
+    (2, 8, 289, 5000, 'mixed'),     # tiles of 1 to 64 rows
+    (3, 3, 500, 64, 'frames'),
+])
+@pytest.mark.parametrize('precision', ['bf16', 'fp32'])
+def test_long_chunks_match_dense_attention(cuda, heads, group, nq, past, tiles, precision):
+    """Long chunks (unpacked keys, causal ranges, merge) against dense float64 attention. bf16: p is
+    rounded to bf16 (8 significant bits: at most 2^-8 of each term) and partial outputs to fp16 (11
+    bits: 2^-11), so an output is within 2^-8 + 2^-10 of the attention over |v| (fp32 sums and
+    exponentials take the rest of 2^-10); fp32: within 1e-3, as every fp32 path. The frame-chunk kernel
+    (path='mfma') must agree with the same bounds, and two calls bit for bit."""
+    announce(f'routes: long chunk heads={heads} group={group} nq={nq} past={past} tiles={tiles} {precision}')
+    assert heads * group * nq >= 4500 and group * nq >= 256
+    case = frame_chunk_case(past, seed=nq + past, heads=heads, q_heads=heads * group, nq=nq)
+    c = GPUCache(None, layers=2, heads=heads, max_tokens=past + nq + 64, precision=precision)
+    g = torch.Generator().manual_seed(past)
+    lengths, t = [], 0
+    while t < past:
+        n = {'ones': 1, 'mixed': int(torch.randint(1, 65, (1,), generator=g))}.get(tiles, 64)
+        lengths.append(min(n, past - t))
+        t += lengths[-1]
+    if past:
+        k, v = (case[x][None].expand(2, -1, -1, -1).contiguous().to(cuda) for x in ('k_hist', 'v_hist'))
+        c.append_batch(k, v, [(4, 8, 16)[i % 3] for i in range(len(lengths))], lengths)
+    q, k, v = (case[x].to(cuda).transpose(0, 1).contiguous().transpose(0, 1)[None] for x in ('q', 'k_new', 'v_new'))
+    starts = torch.zeros(nq, dtype=torch.long)
+    for segments in (None, [0, nq // 3, nq // 3 + 1, nq]):
+        if segments:
+            for b in segments[:-1]:
+                starts[b:] = b
+        ref, mag = _dense(c, case, past, starts, torch.bfloat16 if precision == 'bf16' else torch.float32)
+        bound = mag * (2.0 ** -8 + 2.0 ** -10) + 1e-5 if precision == 'bf16' else torch.full_like(mag, 1e-3)
+        got = c.attend(q, k, v, 0, past, out_dtype=torch.float32, segments=segments)
+        assert bool(((got[0].double() - ref).abs() <= bound).all()), ((got[0].double() - ref).abs() - bound).max()
+        assert torch.equal(got, c.attend(q, k, v, 0, past, out_dtype=torch.float32, segments=segments))
+        assert torch.equal(got.to(torch.bfloat16), c.attend(q, k, v, 0, past, segments=segments))
+        frame = c.attend(q, k, v, 0, past, out_dtype=torch.float32, segments=segments, path='mfma')
+        assert bool(((frame[0].double() - ref).abs() <= bound).all())
+
+
+def test_long_chunk_partials_keep_large_values(cuda):
+    """|V| near the top of bf16: the fp16 partial outputs are stored scaled; V and V * 2^20 give outputs
+    that differ by exactly that factor, up to the one bit a scaled sum may lose (2^-15)."""
+    announce('routes: long chunk, large values')
+    case = frame_chunk_case(2000, seed=9, nq=320)
+    outs = []
+    for scale in (1.0, 2.0 ** 20):
+        c = GPUCache(None, layers=1, heads=5, max_tokens=2400)
+        k, v = case['k_hist'][None].to(cuda), (case['v_hist'].float() * scale).to(torch.bfloat16)[None].to(cuda)
+        c.append_batch(k, v, [16] * 32, [64] * 31 + [16])
+        q, kn, vn = (case[x][None].to(cuda) for x in ('q', 'k_new', 'v_new'))
+        outs.append(c.attend(q, kn, (vn.float() * scale).to(torch.bfloat16), 0, 2000, out_dtype=torch.float32))
+    a, b = outs[0], outs[1] / 2.0 ** 20
+    assert torch.isfinite(b).all()
+    assert (a - b).abs().max() <= 2.0 ** -10 * a.abs().max()
+
+
+def test_long_chunk_without_scratch_for_its_keys(cuda):
+    """dkv_attend_noalloc: the same call as dkv_attend where the unpacked keys and partials fit its
+    scratch buffer; where they do not, the frame-chunk kernel's output instead of a refusal."""
+    import ctypes
+
+    from dkv import _lib
+    announce('routes: long chunk through dkv_attend_noalloc')
+    lib = _lib.load()
+    for nq, past, fits in ((320, 1000, True), (2048, 30000, False)):
+        case = frame_chunk_case(past, seed=nq, nq=nq)
+        c, past = filled(case, cuda, 5)
+        q, k, v = (case[x][None].to(cuda) for x in ('q', 'k_new', 'v_new'))
+        out = torch.empty(1, nq, 15, 64, dtype=torch.float32, device=cuda)
+        a = c.attend_args(q, k, v, 0, past, out)
+        assert (lib.dkv_attend_workspace_bytes(ctypes.byref(a)) <= _lib.DKV_NOALLOC_SCRATCH_BYTES) == fits
+        _lib.check(lib.dkv_attend_noalloc(ctypes.byref(a), _lib.stream_handle(cuda)), 'dkv_attend_noalloc')
+        want = c.attend(q, k, v, 0, past, out_dtype=torch.float32, path='auto' if fits else 'mfma')
+        assert torch.equal(out, want)
