@@ -23,7 +23,7 @@
 // one job. Global loads and stores are 16 bytes per lane over contiguous
 // rows; an LDS transpose hands each lane one whole row, so a row's min/max,
 // scale and reciprocal are computed once.
-#include "dkv_common.h"
+#include "dkv_attn_common.h"
 #include <stdarg.h>
 #include <stdio.h>
 #include <string.h>
@@ -301,6 +301,51 @@ pack_batch_kernel(const dkv_pack_job* __restrict__ jobs, int n_jobs, int wpj, ui
   const int wave = gw - ji * wpj;
   if (j.write_tiles && wave == 0) write_segment_tiles(j, layers, heads, tiles);
   pack_job_wave(j, wave, arena, layers, heads);
+}
+
+// A whole volume, every layer of the tiles in the argument block: a wave packs one (tile, layer, K or
+// V, head), tiles outermost, and the first wave of a tile writes its descriptor. The tile is the
+// whole job, so a volume of 96 tiles x 32 layers needs 96 descriptors in the launch's own arguments
+// where pack_batch_kernel reads 3072 jobs from a table that the host has to build, check and copy
+// (12.9 ms of host time around the 71 us launch); the launch itself takes the same time.
+struct VolumeArgs {
+  const uint16_t *k, *v;  // element (layer, head, token) at its strides; token 0 is first_token
+  int64_t k_layer_stride, k_head_stride, k_tok_stride;
+  int64_t v_layer_stride, v_head_stride, v_tok_stride;
+  uint8_t* arena;
+  dkv_tile* tiles;  // device table from the first tile on
+  int n_tiles, first_token, layers, heads;
+};
+
+__global__ void __launch_bounds__(PACK_THREADS)
+pack_volume_kernel(ArgTiles, VolumeArgs a) {
+  __shared__ __attribute__((aligned(16))) uint8_t stage[PACK_THREADS / 64][WAVE_LDS];
+  uint8_t* lds = stage[(threadIdx.x >> 6)];
+  const int gw = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (PACK_THREADS / 64) + (threadIdx.x >> 6)));
+  const int per_tile = a.layers * 2 * a.heads;
+  const int ti = gw / per_tile;
+  if (ti >= a.n_tiles) return;
+  const int rem = gw - ti * per_tile;
+  const int lk = rem / a.heads, head = rem - lk * a.heads;
+  const int layer = lk >> 1, kv = lk & 1;
+  const uint4 w = arg_tile(ti);
+  const int token_start = (int)w.z, rows = (int)(w.w & 0xffffu), bits = (int)((w.w >> 16) & 0xffu);
+  if (rem == 0 && (threadIdx.x & 63) == 0) *reinterpret_cast<uint4*>(a.tiles + ti) = w;
+  dkv_pack_job j = {};  // the tile as a segment of its own
+  const int64_t t0 = token_start - a.first_token;
+  j.k = a.k + layer * a.k_layer_stride + t0 * a.k_tok_stride;
+  j.v = a.v + layer * a.v_layer_stride + t0 * a.v_tok_stride;
+  j.k_head_stride = a.k_head_stride;
+  j.k_tok_stride = a.k_tok_stride;
+  j.v_head_stride = a.v_head_stride;
+  j.v_tok_stride = a.v_tok_stride;
+  j.seg_offset = (int64_t)((uint64_t)w.y << 32 | w.x);
+  j.seg_rows = j.n = rows;
+  j.layer = layer;
+  j.bits = bits;
+  if (bits == 4) pack_wave<4>(j, kv, head, 0, a.arena, a.layers, a.heads, lds);
+  else if (bits == 8) pack_wave<8>(j, kv, head, 0, a.arena, a.layers, a.heads, lds);
+  else pack_wave<16>(j, kv, head, 0, a.arena, a.layers, a.heads, lds);
 }
 
 // Eight elements of one row after RoPE: y = bf16(bf16(x * cos) + bf16(sign *
@@ -582,6 +627,62 @@ int dkv_pack_batch(const dkv_pack_job* jobs, int32_t n_jobs, int32_t max_n, void
   hipLaunchKernelGGL(pack_batch_kernel, dim3((unsigned)blocks), dim3(PACK_THREADS), 0, (hipStream_t)stream, jobs,
                      n_jobs, wpj, static_cast<uint8_t*>(arena), tiles, layers, heads);
   return (int)hipGetLastError();
+}
+
+int dkv_pack_volume(const void* k, int64_t k_layer_stride, int64_t k_head_stride, int64_t k_tok_stride, const void* v,
+                    int64_t v_layer_stride, int64_t v_head_stride, int64_t v_tok_stride, int32_t tokens,
+                    const dkv_tile* tiles_host, int32_t n_tiles, int32_t first_token, void* arena, int64_t arena_bytes,
+                    dkv_tile* tiles, int32_t layers, int32_t heads, void* stream) {
+  clear_error();
+  if (n_tiles < 0 || layers <= 0 || heads <= 0 || tokens < 0 ||
+      (n_tiles > 0 && (!k || !v || !tiles_host || !arena || !tiles))) {
+    set_error("dkv_pack_volume: bad arguments (n_tiles %d, layers %d, heads %d)", n_tiles, layers, heads);
+    return DKV_EINVAL;
+  }
+  if (!aligned16(k) || !aligned16(v) || !aligned16(tiles) || ((k_layer_stride | k_head_stride | k_tok_stride) & 7) ||
+      ((v_layer_stride | v_head_stride | v_tok_stride) & 7)) {
+    set_error("dkv_pack_volume: K/V must be 16-byte aligned with strides that are multiples of 8 elements");
+    return DKV_EINVAL;
+  }
+  for (int i = 0; i < n_tiles; ++i) {
+    const dkv_tile& t = tiles_host[i];
+    const int64_t at = (int64_t)t.token_start - first_token;
+    if ((t.bits != 4 && t.bits != 8 && t.bits != 16) || t.rows < 1 || t.rows > TILE || at < 0 || at + t.rows > tokens ||
+        t.offset < 0 || (t.offset & 15) || t.offset + slab_bytes(t.rows, t.bits, layers, heads) > arena_bytes) {
+      set_error("dkv_pack_volume: tile %d (offset %lld, token_start %d, rows %d, bits %d) does not lie in the %d tokens "
+                "from %d on and the %lld-byte arena", i, (long long)t.offset, t.token_start, (int)t.rows, (int)t.bits,
+                tokens, first_token, (long long)arena_bytes);
+      return DKV_EINVAL;
+    }
+  }
+  if ((int64_t)DKV_ARG_TILES * layers * 2 * heads > INT32_MAX / 2) {
+    set_error("dkv_pack_volume: %d layers x %d heads exceed one launch", layers, heads);
+    return DKV_EINVAL;
+  }
+  for (int t0 = 0; t0 < n_tiles; t0 += DKV_ARG_TILES) {
+    ArgTiles at;
+    VolumeArgs a;
+    a.k = static_cast<const uint16_t*>(k);
+    a.v = static_cast<const uint16_t*>(v);
+    a.k_layer_stride = k_layer_stride;
+    a.k_head_stride = k_head_stride;
+    a.k_tok_stride = k_tok_stride;
+    a.v_layer_stride = v_layer_stride;
+    a.v_head_stride = v_head_stride;
+    a.v_tok_stride = v_tok_stride;
+    a.arena = static_cast<uint8_t*>(arena);
+    a.tiles = tiles + t0;
+    a.n_tiles = n_tiles - t0 < DKV_ARG_TILES ? n_tiles - t0 : DKV_ARG_TILES;
+    a.first_token = first_token;
+    a.layers = layers;
+    a.heads = heads;
+    for (int i = 0; i < DKV_ARG_TILES; ++i) at.t[i] = i < a.n_tiles ? tiles_host[t0 + i] : dkv_tile{};
+    const int64_t waves = (int64_t)a.n_tiles * layers * 2 * heads;
+    hipLaunchKernelGGL(pack_volume_kernel, dim3((unsigned)((waves + PACK_THREADS / 64 - 1) / (PACK_THREADS / 64))),
+                       dim3(PACK_THREADS), 0, (hipStream_t)stream, at, a);
+    if (hipError_t e = hipGetLastError()) return (int)e;
+  }
+  return 0;
 }
 
 int dkv_rope_pack(const void* qkv, int64_t qkv_row_stride, const void* cos, const void* sin, int64_t cs_row_stride,

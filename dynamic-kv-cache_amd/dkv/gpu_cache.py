@@ -176,6 +176,46 @@ class GPUCache(_CacheBase):
         self.arena_used += need
         return seg
 
+    def _open_segments(self, start, lengths, bits, frame=-1):
+        """_open_segment() of consecutive nonempty segments, all or none: the same bookkeeping, with the
+        tile table filled in one go. Returns the index of the first new tile."""
+        blocks = self.layers * 2 * self.heads
+        n, b = np.array(lengths, dtype=np.int64), np.array(bits, dtype=np.int64)
+        block_of = {w: subblock_bytes(TILE, w) for w in BITS}
+        full_block = np.array([block_of[w] for w in bits], dtype=np.int64)
+        row = full_block // TILE
+        last = (n * row % (TILE * row) + 15) & ~15  # the partial tile's sub-block (0: none)
+        need = (n // TILE * full_block + last) * blocks
+        ends = self.arena_used + np.cumsum(need)
+        counts = (n + TILE - 1) // TILE
+        tile0 = len(self.tile_starts)
+        first = tile0 + np.cumsum(counts) - counts
+        total = int(counts.sum())
+        if tile0 + total > self.tiles.shape[0]:
+            raise ValueError('GPU context limit exceeded')
+        if ends[-1] > self.arena_bytes:  # grown as the segments one by one would have grown it
+            size = self.arena_bytes
+            for e in ends.tolist():
+                if e > size:
+                    size = max(e, ((int(size * 1.5) + 255) // 256) * 256)
+            self._grow(size)
+        starts = start + np.cumsum(n) - n
+        tile = np.arange(total) - np.repeat(first - tile0, counts)  # index within its segment
+        entries = self.tiles_host[tile0:tile0 + total]
+        entries['offset'] = np.repeat(ends - need, counts) + tile * np.repeat(full_block * blocks, counts)
+        entries['token_start'] = np.repeat(starts, counts) + tile * TILE
+        entries['rows'] = np.minimum(np.repeat(n, counts) - tile * TILE, TILE)
+        entries['bits'] = np.repeat(b, counts)
+        entries['reserved'] = 0
+        self.tile_starts.extend(entries['token_start'].tolist())
+        held = self.host_counts
+        for s, w, c, off, t in zip(starts.tolist(), bits, lengths, (ends - need).tolist(), first.tolist()):
+            self.segments.append(_Segment(s, c, w, off, t, frame))
+            self.plan.append((s, s + c, w, held[w]))
+            held[w] += c
+        self.arena_used = int(ends[-1])
+        return tile0
+
     def _grow(self, needed):
         """Grows this cache's arena (forks keep theirs), like the reference's reserve()."""
         size = max(needed, ((int(self.arena_bytes * 1.5) + 255) // 256) * 256)
@@ -401,17 +441,25 @@ class GPUCache(_CacheBase):
 
         k, v: [layers, heads, sum(lengths), 64] bf16 device tensors (last dim contiguous).
         bits, lengths: width and token count of each segment, in order. Equivalent to calling
-        select(bits[i]) and append() for every layer and segment; returns the history length
-        before the batch. Returns a PackBatch that can re-run the same launch (benchmarks).
+        select(bits[i]) and append() for every layer and segment. Returns a PackVolume (online
+        caches) or a PackBatch (planned ones) that can re-run the same launch (benchmarks).
         """
         if k.shape[0] != self.layers or k.shape[1] != self.heads or k.shape[-1] != self.dim or k.device.type != 'cuda':
             raise ValueError('append_batch expects [layers, heads, tokens, 64] CUDA tensors')
         if sum(lengths) != k.shape[2] or len(bits) != len(lengths) or len(set(self.seen)) != 1:
             raise ValueError('append_batch: lengths must cover the tokens and every layer must be level')
+        if v.dim() != 4 or v.shape[-1] != self.dim or not v.is_cuda or any(a < b for a, b in zip(v.shape, k.shape)):
+            raise ValueError('append_batch expects v of the shape of k')
         past = self.seen[0]
         if past + k.shape[2] > self.capacity:
             raise ValueError('GPU context limit exceeded')
         k, v = self._kv_view4(k), self._kv_view4(v)
+        if self.online and lengths and min(lengths) > 0:
+            tile0 = self._open_segments(past, lengths, bits, self.frame_id)
+            batch = PackVolume(self, k, v, past, tile0)
+            batch.run()
+            self.seen = [past + k.shape[2]] * self.layers
+            return batch
         jobs = []
         start = past
         for b, n in zip(bits, lengths):
@@ -1019,6 +1067,24 @@ class SegmentBatch:
                                                  self.direction, c.arena.data_ptr(), c.arena_bytes,
                                                  c.tiles.data_ptr(), c.layers, c.heads,
                                                  _lib.stream_handle(c.device)), 'dkv_segment_batch')
+
+
+class PackVolume:
+    """dkv_pack_volume over the tiles of a cache from tile0 on: every layer of k, v [layers, heads,
+    tokens, 64]. run() relaunches it."""
+
+    def __init__(self, cache, k, v, first_token, tile0):
+        self.cache, self.k, self.v, self.first_token, self.tile0 = cache, k, v, first_token, tile0
+        self.tiles_host = cache.tiles_host[tile0:len(cache.tile_starts)].copy()  # (a reset cache reuses its own)
+        self.arena, self.arena_bytes, self.tiles = cache.arena, cache.arena_bytes, cache.tiles
+
+    def run(self):
+        c, k, v = self.cache, self.k, self.v
+        _lib.check(_lib.load().dkv_pack_volume(
+            k.data_ptr(), k.stride(0), k.stride(1), k.stride(2), v.data_ptr(), v.stride(0), v.stride(1), v.stride(2),
+            k.shape[2], self.tiles_host.ctypes.data, len(self.tiles_host), self.first_token, self.arena.data_ptr(),
+            self.arena_bytes, self.tiles.data_ptr() + 16 * self.tile0, c.layers, c.heads,
+            _lib.raw_stream(c.device)), 'dkv_pack_volume')
 
 
 class PackBatch:

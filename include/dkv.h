@@ -169,6 +169,20 @@ int dkv_pack_batch(const dkv_pack_job* jobs, int32_t n_jobs, int32_t max_n,
                    void* arena, int64_t arena_bytes, dkv_tile* tiles,
                    int32_t layers, int32_t heads, void* stream);
 
+/* Pack every layer of a volume of new tokens, one launch per DKV_ARG_TILES tiles:
+ * k and v are bf16 views [layers, heads, tokens, 64] (element strides, contiguous
+ * last dimension), tiles_host a HOST array of the n_tiles whole tiles they fill
+ * (token_start counts from first_token; checked against tokens and the arena).
+ * The bytes are what dkv_pack of every (tile, layer) writes; tiles, the DEVICE
+ * table from the first of these tiles on, receives the descriptors. Unlike
+ * dkv_pack_batch it needs no job table in device memory. No reference
+ * counterpart (see dkv_pack_batch). */
+int dkv_pack_volume(const void* k, int64_t k_layer_stride, int64_t k_head_stride, int64_t k_tok_stride,
+                    const void* v, int64_t v_layer_stride, int64_t v_head_stride, int64_t v_tok_stride,
+                    int32_t tokens, const dkv_tile* tiles_host, int32_t n_tiles, int32_t first_token,
+                    void* arena, int64_t arena_bytes, dkv_tile* tiles, int32_t layers, int32_t heads,
+                    void* stream);
+
 /* Checks a HOST copy of a job table against the arena (what dkv_pack checks for
  * one job), so that a table can be validated before it is copied to the device
  * and launched with dkv_pack_batch. No reference counterpart (see dkv_pack_batch). */

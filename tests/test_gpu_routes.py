@@ -201,3 +201,44 @@ def test_long_chunk_without_scratch_for_its_keys(cuda):
         _lib.check(lib.dkv_attend_noalloc(ctypes.byref(a), _lib.stream_handle(cuda)), 'dkv_attend_noalloc')
         want = c.attend(q, k, v, 0, past, out_dtype=torch.float32, path='auto' if fits else 'mfma')
         assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize('layers,heads,lengths', [
+    (3, 5, [64, 64, 64]), (2, 3, [1, 63, 65, 130, 7]), (1, 1, [64] * 128 + [5]), (2, 2, [1] * 300),
+    (4, 8, [200]),
+])
+@pytest.mark.parametrize('strided', [False, True])
+def test_volume_append_equals_appends(cuda, layers, heads, lengths, strided):
+    """append_batch of an online cache (descriptors in the launch's argument block, 128 tiles a launch)
+    writes the bytes, the tile table and the bookkeeping that an append per layer and segment writes,
+    also behind earlier segments and for K/V whose tokens or heads are further apart."""
+    announce(f'routes: volume append layers={layers} heads={heads} segments={len(lengths)} strided={strided}')
+    n = sum(lengths)
+    bits = [(4, 8, 16)[i % 3] for i in range(len(lengths))]
+    g = torch.Generator().manual_seed(n + heads)
+    k, v = (torch.randn((layers, heads, n + 3, 64), generator=g).to(torch.bfloat16).to(cuda) for _ in range(2))
+    if strided:
+        k = k.permute(2, 0, 1, 3).contiguous().permute(1, 2, 0, 3)  # tokens outermost
+        v = torch.cat((v, v), -1)[..., :64]
+    a, b = (GPUCache(None, layers=layers, heads=heads, max_tokens=n + 3) for _ in range(2))
+    for c in (a, b):
+        c.arena.zero_()
+        for layer in range(layers):
+            c.select(8, 4)
+            c.append(k[None, layer, :, :3], v[None, layer, :, :3], layer)
+    batch = a.append_batch(k[:, :, 3:], v[:, :, 3:], bits, lengths)
+    t = 3
+    for w, m in zip(bits, lengths):
+        b.select(w, 4)
+        for layer in range(layers):
+            b.append(k[None, layer, :, t:t + m], v[None, layer, :, t:t + m], layer)
+        t += m
+    assert a.seen == b.seen and a.plan == b.plan and a.arena_used == b.arena_used
+    used = a.arena_used
+    assert torch.equal(a.arena[:used], b.arena[:used])
+    tiles = len(a.tile_starts)
+    assert torch.equal(a.tiles[:tiles], b.tiles[:tiles]) and a.tiles_host[:tiles].tobytes() == \
+        a.tiles[:tiles].cpu().numpy().tobytes()
+    a.arena[a.segments[1].offset:].zero_()
+    batch.run()
+    assert torch.equal(a.arena[:used], b.arena[:used])
