@@ -607,10 +607,11 @@ attn_mfma_kernel(typename std::conditional<ARGT, ArgTiles, NoArgTiles>::type, dk
   struct Raw {
     uint4 k[PN], v[PN];
   };
-  auto load = [&](int rel, Raw& r) {
+  auto load_unit = [&](const Unit& un, Raw& r) {
 #pragma unroll
-    for (int i = 0; i < PN; ++i) raw_load(a, unit(rel), h, lt + 256 * i, r.k[i], r.v[i]);
+    for (int i = 0; i < PN; ++i) raw_load(a, un, h, lt + 256 * i, r.k[i], r.v[i]);
   };
+  auto load = [&](int rel, Raw& r) { load_unit(unit(rel), r); };
   // The zeros of a Raw, made opaque where they are written (the kernel's start): the compiler
   // would otherwise move them down to the loads, and each move brings back the wait described at
   // raw_load.
@@ -630,23 +631,30 @@ attn_mfma_kernel(typename std::conditional<ARGT, ArgTiles, NoArgTiles>::type, dk
     }
   };
   if constexpr (SMALL) {
-    // One buffer: per unit, load, stage, dequantize and compute, with a barrier after the
-    // staging and one after the dequantization. The default plan gives each workgroup one unit;
-    // graph replays over longer histories may give it more, whose loads then wait for the unit
-    // before (no registers held across the MFMA work: four workgroups per CU need <= 128 VGPRs).
+    // One buffer of raw bytes and tiles: per unit, stage, dequantize and compute, with a barrier after
+    // the staging and one after the dequantization. Up to the number of workgroups that are resident
+    // at once the default plan gives each one unit; longer histories, and graph replays, give it
+    // more, and unit i + 1's loads go out as soon as unit i's bytes have left the registers, not after
+    // its MFMA work (one token, us per call: 8 KV heads past 33957, five units each, 21.2 -> 18.9;
+    // 5 KV heads, 4 tokens past 30000 16.4 -> 15.3; one unit each, past 8128, the same). Four
+    // workgroups per CU leave 128 VGPRs, too few for a second unit in flight.
     Raw r = {};
     opaque(r);
+    Unit un = unit(0);
+    load_unit(un, r);
     for (int i = 0; i < n; ++i) {
-      load(i, r);
       if (i) __syncthreads();  // unit i - 1's MFMA work is done with the tiles
       stage(0, r);
+      const Unit next = unit(min(i + 1, n - 1));
+      if (i + 1 < n) load_unit(next, r);
       if (i == 0) DKV_TL(tl_mfma, 1);
       __syncthreads();
-      dequant(unit(i), 0, 0);
+      dequant(un, 0, 0);
       if (i == 0) DKV_TL(tl_mfma, 2);
       __syncthreads();
-      compute(unit(i), 0, i == 0);
+      compute(un, 0, i == 0);
       if (i == 0) DKV_TL(tl_mfma, 3);
+      un = next;
     }
   } else {
     Raw r = {}, r0 = {}, r2 = {};

@@ -166,6 +166,36 @@ def test_long_chunks_match_dense_attention(cuda, heads, group, nq, past, tiles, 
         assert bool(((frame[0].double() - ref).abs() <= bound).all())
 
 
+@pytest.mark.parametrize('heads,group,nq,past,tiles', [
+    (32, 3, 1, 2500, 'frames'),    # 41 units at 32 KV heads: two per workgroup by default, descriptors in the arguments
+    (5, 3, 10, 1999, 'mixed'),     # 30 rows; tiles of 1 to 64 rows
+    (8, 2, 1, 700, 'ones'),        # 700 tiles: the device table, more units in a range than its window of 64
+    (1, 8, 4, 64, 'frames'),       # one tile and the chunk
+])
+def test_decode_workgroups_of_several_units(cuda, heads, group, nq, past, tiles):
+    """Few query rows at precision 0 when a workgroup walks several units (each loaded while the one
+    before it is worked on), by default and at given split counts: within the bounds of
+    test_long_chunks_match_dense_attention of dense float64 attention."""
+    announce(f'routes: decode units heads={heads} group={group} nq={nq} past={past} tiles={tiles}')
+    assert group * nq <= 32
+    case = frame_chunk_case(past, seed=past, heads=heads, q_heads=heads * group, nq=nq)
+    c = GPUCache(None, layers=1, heads=heads, max_tokens=past + nq + 64, precision='bf16')
+    g = torch.Generator().manual_seed(past)
+    lengths, t = [], 0
+    while t < past:
+        n = {'ones': 1, 'mixed': int(torch.randint(1, 65, (1,), generator=g))}.get(tiles, 64)
+        lengths.append(min(n, past - t))
+        t += lengths[-1]
+    c.append_batch(case['k_hist'][None].to(cuda), case['v_hist'][None].to(cuda),
+                   [(4, 8, 16)[i % 3] for i in range(len(lengths))], lengths)
+    q, k, v = (case[x][None].to(cuda) for x in ('q', 'k_new', 'v_new'))
+    ref, mag = _dense(c, case, past, torch.zeros(nq, dtype=torch.long), torch.bfloat16)
+    bound = mag * (2.0 ** -8 + 2.0 ** -10) + 1e-5
+    for splits in (0, 1, 2, 7, len(lengths)):
+        got = c.attend(q, k, v, 0, past, out_dtype=torch.float32, splits=splits)
+        assert bool(((got[0].double() - ref).abs() <= bound).all()), splits
+
+
 def test_long_chunk_partials_keep_large_values(cuda):
     """|V| near the top of bf16: the fp16 partial outputs are stored scaled; V and V * 2^20 give outputs
     that differ by exactly that factor, up to the one bit a scaled sum may lose (2^-15)."""
