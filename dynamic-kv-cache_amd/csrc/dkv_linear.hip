@@ -10,7 +10,9 @@
 //             o_proj and down_proj;
 //             silu_mul: w holds [gate | up] rows (2 * inter of them) and
 //             out[:, c] = bf16(bf16(silu(bf16(g_c))) * bf16(u_c))
-//             (src/gpu_ops.py:14-17, 23-25).
+//             (src/gpu_ops.py:14-17, 23-25);
+//             rope: w holds the joined [q | k | v] heads of 64 rows; RoPE on q and k, the q, k and v
+//             blocks, and K and V packed into a segment (dkv_rope_pack's work and bytes).
 //
 // The chunks are 1-100 rows, so the weights (1.8-9.8 MB per projection of the
 // 960-wide decoder) dominate the traffic: the kernel is a weight stream. A
@@ -24,6 +26,7 @@
 // numbers its tiles so that the row blocks sharing a weight tile land on one
 // XCD (one L2).
 #include "dkv_common.h"
+#include "dkv_rope_pack.h"
 
 namespace dkv {
 namespace {
@@ -36,7 +39,7 @@ union Op8 {
   u32x4 u;
 };
 
-enum { EPI_PLAIN = 0, EPI_RESIDUAL = 1, EPI_SILU_MUL = 2 };
+enum { EPI_PLAIN = 0, EPI_RESIDUAL = 1, EPI_SILU_MUL = 2, EPI_ROPE = 3 };
 
 struct LinearArgs {  // passed by value and never written (a written copy would go to scratch)
   const uint16_t* x;
@@ -54,6 +57,21 @@ struct LinearArgs {  // passed by value and never written (a written copy would 
   int row_groups;   // ceil(rows / (16 * RB))
   int up;           // n_out (EPI_SILU_MUL: the first weight row of the up half)
   int layout;       // LAYOUT_* bits: which of w, x and out are MFMA-tiled
+};
+
+struct NoRope {};
+struct RopeArgs {  // EPI_ROPE: what dkv_rope_pack takes after the projection
+  const uint16_t* cosv;
+  const uint16_t* sinv;
+  int64_t cs_stride;
+  uint16_t* q_out;
+  uint16_t* k_out;
+  uint16_t* v_out;
+  dkv_pack_job hjob;
+  const dkv_pack_job* djob;  // read in place of hjob unless null
+  uint8_t* arena;
+  dkv_tile* tiles;
+  int q_heads, heads, layers;
 };
 
 // Operand layouts. Rows of k contiguous elements, or MFMA-tiled: the 16 rows x 64 k of one pair
@@ -81,8 +99,8 @@ __device__ __forceinline__ float lane_group_sum(float x) {
   return __uint_as_float(q[0]) + __uint_as_float(q[1]);
 }
 
-template <int CH, int NT, int WAVES, int RB, int EPI, bool NORM, int OPS>
-__global__ void __launch_bounds__(64 * WAVES) linear_kernel(const LinearArgs a) {
+template <int CH, int NT, int WAVES, int RB, int EPI, bool NORM, int OPS, typename Rope>
+__device__ __forceinline__ void linear_body(const LinearArgs& a, const Rope& rope) {
   constexpr int NB = EPI == EPI_SILU_MUL ? 2 * NT : NT;  // column blocks multiplied
   // The arguments the first loads depend on, read together (placed by their uses, the compiler
   // read them in two dependent rounds of scalar loads, each a round trip to the cache hierarchy).
@@ -136,6 +154,20 @@ __global__ void __launch_bounds__(64 * WAVES) linear_kernel(const LinearArgs a) 
       resv[o] = *reinterpret_cast<const uint2*>(
           a.res + ((a.layout & LAYOUT_RES_TILED) ? tiled_offset((rg * RB + o / NT) * 16 + col, c, a.up >> 6)
                                                  : (int64_t)row * a.ldr + c));
+    }
+  }
+
+  // EPI_ROPE: cos, sin and the job of the 8 rows that waves 0 and 1 finish each, 8 lanes per row.
+  // (Read here, the job arrives with the operands; read where it is used it was one more round trip.)
+  u32x4 cs = {0, 0, 0, 0}, sn = cs;
+  dkv_pack_job job = {};
+  if constexpr (EPI == EPI_ROPE) {
+    job = rope.djob ? *rope.djob : rope.hjob;
+    asm volatile("" ::: "memory");
+    if (wave < 2) {
+      const int64_t o = (int64_t)min(rg * 16 + 8 * wave + (lane >> 3), a.rows - 1) * rope.cs_stride + 8 * (lane & 7);
+      cs = *reinterpret_cast<const u32x4*>(rope.cosv + o);
+      sn = *reinterpret_cast<const u32x4*>(rope.sinv + o);
     }
   }
 
@@ -291,6 +323,26 @@ __global__ void __launch_bounds__(64 * WAVES) linear_kernel(const LinearArgs a) 
       else usum[o] = s;
     }
   }
+  if constexpr (EPI == EPI_ROPE) {
+    // The workgroup holds 16 whole rows of one 64-wide head: rounded to bf16 they meet in LDS, and
+    // two waves rotate and pack 8 rows each.
+    static_assert(NT == 4 && RB == 1, "one head per workgroup");
+    constexpr int RS = D + 8;  // LDS row, in elements
+    __shared__ __attribute__((aligned(16))) uint16_t head_rows[16 * RS];
+#pragma unroll
+    for (int o = 0; o < OUT; ++o) {
+      if (o % WAVES != wave) continue;
+      *reinterpret_cast<uint2*>(head_rows + col * RS + 16 * o + 4 * g) =
+          make_uint2(pack_bf16(gsum[o][0], gsum[o][1]), pack_bf16(gsum[o][2], gsum[o][3]));
+    }
+    __syncthreads();
+    if (wave >= 2) return;
+    const int r = 8 * wave + (lane >> 3), c = lane & 7, tok = rg * 16 + r;
+    if (ct == 0 && rg == 0 && wave == 0 && job.write_tiles) write_segment_tiles(job, rope.layers, rope.heads, rope.tiles);
+    rope_pack_row(*reinterpret_cast<const u32x4*>(head_rows + r * RS + 8 * c), cs, sn, ct, tok, tok < a.rows, c, a.rows,
+                  rope.q_heads, rope.q_out, rope.k_out, rope.v_out, job, rope.arena, rope.layers, rope.heads);
+    return;
+  }
 #pragma unroll
   for (int o = 0; o < OUT; ++o) {
     if (o % WAVES != wave) continue;
@@ -315,6 +367,23 @@ __global__ void __launch_bounds__(64 * WAVES) linear_kernel(const LinearArgs a) 
     uint16_t* dst = a.out + ((a.layout & LAYOUT_OUT_TILED) ? tiled_offset(row, c, a.up >> 6) : (int64_t)row * a.ldo + c);
     *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3]));
   }
+}
+
+template <int CH, int NT, int WAVES, int RB, int EPI, bool NORM, int OPS>
+__global__ void __launch_bounds__(64 * WAVES) linear_kernel(const LinearArgs a) {
+  linear_body<CH, NT, WAVES, RB, EPI, NORM, OPS>(a, NoRope{});
+}
+
+// Q/K/V with the RMSNorm prologue that ends in dkv_rope_pack's work: a workgroup computes 16 rows of one
+// 64-wide head, so the rows it rotates and quantizes are its own. Half as many workgroups as the plain
+// projection, each with twice the weight bytes (123 KB at k 960, which bounds it), but one launch and one
+// round trip of q | k | v through memory less: the 960-wide decoder's launch 7.2 us instead of 5.6 + 3.5
+// at 64 rows. A whole layer past 640 in graph replays, two launches -> one: 1 row 25.6 -> 25.0 us,
+// 16 rows 28.2 -> 27.1, 64 rows 32.4 -> 31.1, 128 rows 42.6 -> 39.5, 256 rows 56.5 -> 54.0, 340 rows
+// 64.0 -> 62.1: better at every size that keeps the few-row kernel.
+template <int CH, int OPS>
+__global__ void __launch_bounds__(512) linear_rope_kernel(const LinearArgs a, const RopeArgs rope) {
+  linear_body<CH, 4, 8, 1, EPI_ROPE, true, OPS>(a, rope);
 }
 
 // The same projections for many rows (prompts, several frames at once), where linear_kernel reads
@@ -725,6 +794,70 @@ int dkv_linear_tiled(const void* x, int64_t x_row_stride, const void* w, int64_t
   else if (epilogue == EPI_RESIDUAL)
     norm ? launch_epi<EPI_RESIDUAL, true>(s, a, st) : launch_epi<EPI_RESIDUAL, false>(s, a, st);
   else norm ? launch_epi<EPI_SILU_MUL, true>(s, a, st) : launch_epi<EPI_SILU_MUL, false>(s, a, st);
+  return (int)hipGetLastError();
+}
+
+int dkv_linear_rope_pack(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride, int32_t n, int32_t k,
+                         const void* norm_weight, float eps, int32_t layout, const void* cos, const void* sin,
+                         int64_t cs_row_stride, int32_t q_heads, void* q_out, void* k_out, void* v_out,
+                         const dkv_pack_job* job, int32_t job_on_device, void* arena, int64_t arena_bytes,
+                         dkv_tile* tiles, int32_t layers, int32_t heads, void* stream) {
+  clear_error();
+  const bool wt = layout & LAYOUT_W_TILED;
+  if (!x || !w || !norm_weight || !cos || !sin || !q_out || !k_out || !v_out || !job || !arena || !tiles || n < 1 ||
+      k <= 0 || (k & 63) || k > 64 * 8 * MAX_NORM_CH || q_heads <= 0 || heads <= 0 || layers <= 0 ||
+      (layout & ~LAYOUT_W_TILED) || !al16(x) || !al16(w) || !al16(norm_weight) || !al16(cos) || !al16(sin) ||
+      !al16(q_out) || !al16(k_out) || !al16(v_out) || (x_row_stride & 7) || x_row_stride < k ||
+      (!wt && ((w_row_stride & 7) || w_row_stride < k)) || (cs_row_stride & 7) || cs_row_stride < D) {
+    set_error("dkv_linear_rope_pack: bad arguments (%d rows of %d; at least one row, k a multiple of 64 up to %d, 16-byte "
+              "aligned bf16 buffers, strides multiples of 8 elements)", n, k, 64 * 8 * MAX_NORM_CH);
+    return DKV_EINVAL;
+  }
+  if (!job_on_device) {
+    if (int rc = check_job(*job, arena_bytes, layers, heads)) return rc;
+    if (job->n != n || (job->write_tiles && job->tile_index0 < 0)) {
+      set_error("dkv_linear_rope_pack: the job appends %d tokens, the projection has %d (or a negative tile index)",
+                job->n, n);
+      return DKV_EINVAL;
+    }
+  }
+  LinearArgs a = {};
+  a.x = static_cast<const uint16_t*>(x);
+  a.ldx = x_row_stride;
+  a.w = static_cast<const uint16_t*>(w);
+  a.ldw = w_row_stride;
+  a.norm = static_cast<const uint16_t*>(norm_weight);
+  a.eps = eps;
+  a.rows = n;
+  a.k = k;
+  a.kp = k / 64;
+  a.n_tiles = q_heads + 2 * heads;
+  a.row_groups = (n + 15) / 16;
+  a.up = a.n_tiles * D;
+  a.layout = layout;
+  RopeArgs r;
+  r.cosv = static_cast<const uint16_t*>(cos);
+  r.sinv = static_cast<const uint16_t*>(sin);
+  r.cs_stride = cs_row_stride;
+  r.q_out = static_cast<uint16_t*>(q_out);
+  r.k_out = static_cast<uint16_t*>(k_out);
+  r.v_out = static_cast<uint16_t*>(v_out);
+  r.hjob = job_on_device ? dkv_pack_job{} : *job;
+  r.djob = job_on_device ? job : nullptr;
+  r.arena = static_cast<uint8_t*>(arena);
+  r.tiles = tiles;
+  r.q_heads = q_heads;
+  r.heads = heads;
+  r.layers = layers;
+  const dim3 grid((unsigned)((a.n_tiles + 7) / 8) * 8u * (unsigned)a.row_groups);
+  hipStream_t st = (hipStream_t)stream;
+  if (a.kp <= 8) {
+    if (wt) hipLaunchKernelGGL((linear_rope_kernel<1, LAYOUT_W_TILED>), grid, dim3(512), 0, st, a, r);
+    else hipLaunchKernelGGL((linear_rope_kernel<1, 0>), grid, dim3(512), 0, st, a, r);
+  } else {
+    if (wt) hipLaunchKernelGGL((linear_rope_kernel<2, LAYOUT_W_TILED>), grid, dim3(512), 0, st, a, r);
+    else hipLaunchKernelGGL((linear_rope_kernel<2, 0>), grid, dim3(512), 0, st, a, r);
+  }
   return (int)hipGetLastError();
 }
 

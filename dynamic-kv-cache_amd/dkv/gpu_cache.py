@@ -391,7 +391,18 @@ class GPUCache(_CacheBase):
         self.seen[layer] = past + n
         return q, k, v, past
 
-    def _fused_attention(self, n, q_heads, layer, qkv, qkv_stride, cos, sin, cs_stride, qkv_out, out, stream):
+    def append_hidden(self, x, weight, weight_stride, norm, eps, layout, cos, sin, q_heads, layer):
+        """append_projection of the joined Q/K/V projection of RMSNorm(x), projection included
+        (dkv_linear_rope_pack), for the recorded launches of graph steps: (q, k, v, past). The caller
+        has checked what that entry asks for: x [n, k], cos and sin [n, 64] bf16 rows, n >= 1."""
+        n = x.shape[0]
+        q = x.new_empty((1, q_heads, n, 64))
+        k, v = (x.new_empty((1, self.heads, n, 64)) for _ in range(2))
+        project = (x.data_ptr(), x.stride(0), weight.data_ptr(), weight_stride, n, x.shape[1], norm.data_ptr(), eps, layout)
+        return q, k, v, self._graph.append_hidden(project, cos, sin, q_heads, layer, q, k, v)
+
+    def _fused_attention(self, n, q_heads, layer, qkv, qkv_stride, cos, sin, cs_stride, qkv_out, out, stream,
+                         project=None):
         """append_projection() then attend() for the fused decoder layer's eager launches: the same
         two launches with the same arguments (so the same bytes and outputs), without the per-call
         checks of the general entry points, which cost more host time than the GPU spends on a
@@ -408,9 +419,14 @@ class GPUCache(_CacheBase):
         job = _lib.PackJob(kp, vp, head, d, head, d, seg.offset, seg.rows, seg.start, past - seg.start,
                            n, layer, seg.bits, seg.tile0, write_tiles)
         lib = _lib.load()
-        _lib.check(lib.dkv_rope_pack(qkv, qkv_stride, cos, sin, cs_stride, n, q_heads, qkv_out, kp, vp,
-                                     ctypes.byref(job), 0, self.arena.data_ptr(), self.arena_bytes,
-                                     self.tiles.data_ptr(), self.layers, H, stream), 'dkv_rope_pack')
+        if project is not None:
+            _lib.check(lib.dkv_linear_rope_pack(*project, cos, sin, cs_stride, q_heads, qkv_out, kp, vp,
+                                                ctypes.byref(job), 0, self.arena.data_ptr(), self.arena_bytes,
+                                                self.tiles.data_ptr(), self.layers, H, stream), 'dkv_linear_rope_pack')
+        else:
+            _lib.check(lib.dkv_rope_pack(qkv, qkv_stride, cos, sin, cs_stride, n, q_heads, qkv_out, kp, vp,
+                                         ctypes.byref(job), 0, self.arena.data_ptr(), self.arena_bytes,
+                                         self.tiles.data_ptr(), self.layers, H, stream), 'dkv_rope_pack')
         self.seen[layer] = past + n
         a = self._fused_args
         if a is None or self._fused_key != (n, q_heads):
@@ -954,6 +970,20 @@ class GraphSteps:
         _lib.check(_lib.load().dkv_pack_batch(self.dev.data_ptr() + layer * self.job_bytes, 1, self.chunk,
                                               c.arena.data_ptr(), c.arena_bytes, c.tiles.data_ptr(), c.layers,
                                               c.heads, _lib.stream_handle(c.device)), 'dkv_pack_batch')
+        return self.state[0]
+
+    def append_hidden(self, project, cos, sin, q_heads, layer, q, k, v):
+        c = self.cache
+        if self.state is None:
+            raise ValueError('graph_step() must run before the recorded append')
+        if k.shape[2] != self.chunk:
+            raise ValueError(f'graph steps were set up for {self.chunk}-token chunks, got {k.shape[2]}')
+        self.kv[layer] = (k, v)
+        self.kv_version += 1
+        _lib.check(_lib.load().dkv_linear_rope_pack(
+            *project, cos.data_ptr(), sin.data_ptr(), cos.stride(0), q_heads, q.data_ptr(), k.data_ptr(), v.data_ptr(),
+            self.dev.data_ptr() + layer * self.job_bytes, 1, c.arena.data_ptr(), c.arena_bytes, c.tiles.data_ptr(),
+            c.layers, c.heads, _lib.stream_handle(c.device)), 'dkv_linear_rope_pack')
         return self.state[0]
 
     def append_projection(self, qkv, cos, sin, q_heads, layer, q, k, v):

@@ -217,7 +217,7 @@ class _LayerPlan:
     epsilons and the head counts."""
     __slots__ = ('qkv_w', 'o_w', 'gu_w', 'd_w', 'ln1_w', 'ln2_w', 'qkv_args', 'o_args', 'gu_args', 'd_args',
                  'eps1', 'eps2', 'q_heads', 'kv_heads', 'eager_ok', 'layer_idx', 'width', 'inter', 'norm1_apart',
-                 'norm2_apart')
+                 'norm2_apart', 'rope_in_qkv')
 
     def holds(self, layer):
         # the modules' own dicts: nn.Module attribute lookups cost more than the rest of this check
@@ -300,6 +300,8 @@ def _layer_plan(layer, n, width):
     # many rows: the norms as launches of their own, before Q/K/V and gate/up
     p.norm1_apart = _prenorm(n, p.qkv_w.shape[0], width, LINEAR_PLAIN)
     p.norm2_apart = _prenorm(n, p.gu_w.shape[0], width, LINEAR_SILU_MUL)
+    # otherwise Q/K/V goes on to RoPE and the pack in its own launch (faster at every such size)
+    p.rope_in_qkv = p.eager_ok and n > 0 and not p.norm1_apart
     plans[(n, width)] = p
     return p
 
@@ -347,10 +349,14 @@ def _fused_layer_eager(p, tiles, h, n, cache, cos, sin):
     if p.norm1_apart:
         _lib.check(lib.dkv_rms_norm_tiled(xp, width, norm1, xn, n, width, p.eps1, 0, stream), 'dkv_rms_norm_tiled')
         qx, norm1, ql = xn, None, ql | LINEAR_X_TILED
-    _lib.check(lib.dkv_linear_tiled(qx, width, qw.data_ptr(), qld, n, qrows, qk, norm1, p.eps1,
-                                    LINEAR_PLAIN, None, 0, qkv, qrows, ql, stream), 'dkv_linear')
+    project = None
+    if p.rope_in_qkv:  # RoPE and the pack in the projection's launch
+        project = (qx, width, qw.data_ptr(), qld, n, qk, norm1, p.eps1, ql)
+    else:
+        _lib.check(lib.dkv_linear_tiled(qx, width, qw.data_ptr(), qld, n, qrows, qk, norm1, p.eps1,
+                                        LINEAR_PLAIN, None, 0, qkv, qrows, ql, stream), 'dkv_linear')
     cache._fused_attention(n, p.q_heads, p.layer_idx, qkv, qrows, cos.data_ptr(), sin.data_ptr(), cos.stride(0),
-                           base + 2 * o_qkvo, att, stream)
+                           base + 2 * o_qkvo, att, stream, project)
     _lib.check(lib.dkv_linear_tiled(att, ok, ow.data_ptr(), old, n, orows, ok, None, 1e-6, LINEAR_RESIDUAL, xp,
                                     width, h2, orows, ol, stream), 'dkv_linear')
     gx, norm2 = h2, p.ln2_w.data_ptr()
@@ -366,7 +372,7 @@ def _fused_layer_eager(p, tiles, h, n, cache, cos, sin):
 
 
 def fused_decoder_layer(layer, hidden_states, cache, position_embeddings):
-    """One LlamaDecoderLayer forward on a packed GPUCache as six launches plus the attention's
+    """One LlamaDecoderLayer forward on a packed GPUCache as four or five launches plus the attention's
     two; None when the layer, the inputs or the cache are outside what they cover. What depends
     only on the layer and the chunk length is checked once (_layer_plan); eager launches on
     contiguous inputs then take _fused_layer_eager, and graph captures the general path below."""
@@ -392,8 +398,22 @@ def fused_decoder_layer(layer, hidden_states, cache, position_embeddings):
     o_w, d_w = attn.o_proj.weight, mlp.down_proj.weight
     x = h.reshape(n, width)
     qt, ot, gt, dt = tiles if tiles is not None else (None,) * 4
-    qkv = linear(x, attn._qkv_weight, norm=ln1.weight, eps=ln1.variance_epsilon, weight_tiled=qt)
-    o = attend_projection(attn, cache, qkv.view(1, n, -1), position_embeddings)
+    packed = None
+    if p.rope_in_qkv and p.kv_heads == cache.heads and cache._graph is not None:
+        cos, sin = position_embeddings
+        if (x.stride(-1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and cos.shape == (1, n, 64)
+                and sin.shape == cos.shape and all(t.is_cuda and t.dtype == torch.bfloat16 and t.stride(-1) == 1
+                                                   and t.stride(1) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (cos, sin))
+                and cos.stride(1) == sin.stride(1)):
+            w, layout = (qt, LINEAR_W_TILED) if qt is not None else (p.qkv_w, 0)
+            packed = cache.append_hidden(x, w, w.stride(0), ln1.weight, p.eps1, layout, cos[0], sin[0], p.q_heads,
+                                         p.layer_idx)
+    if packed is not None:
+        q, k, v, past = packed
+        o = cache.attend(q, k, v, p.layer_idx, past)
+    else:
+        qkv = linear(x, attn._qkv_weight, norm=ln1.weight, eps=ln1.variance_epsilon, weight_tiled=qt)
+        o = attend_projection(attn, cache, qkv.view(1, n, -1), position_embeddings)
     # SiLU*up to down_proj, and h2 to gate/up and down_proj, in the tiled layout
     act_tiled = tiles is not None and p.inter % 64 == 0
     h2_tiled = tiles is not None and width % 64 == 0

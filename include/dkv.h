@@ -350,6 +350,15 @@ int dkv_linear_tiled(const void* x, int64_t x_row_stride, const void* w, int64_t
                      int32_t epilogue, const void* residual, int64_t residual_row_stride,
                      void* out, int64_t out_row_stride, int32_t layout, void* stream);
 
+/* dkv_linear with the RMSNorm prologue over the joined [q | k | v] weight (k columns, (q_heads + 2 heads) * 64
+ * rows), then dkv_rope_pack on the result, in one launch: the same q_out, k_out, v_out and packed bytes. x has n >= 1
+ * rows of k (a multiple of 64, at most 1024); layout is 0 or DKV_LINEAR_W_TILED; the rest as those two take it. */
+int dkv_linear_rope_pack(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride, int32_t n, int32_t k,
+                         const void* norm_weight, float eps, int32_t layout, const void* cos, const void* sin,
+                         int64_t cs_row_stride, int32_t q_heads, void* q_out, void* k_out, void* v_out,
+                         const dkv_pack_job* job, int32_t job_on_device, void* arena, int64_t arena_bytes,
+                         dkv_tile* tiles, int32_t layers, int32_t heads, void* stream);
+
 /* RMSNorm of x rows [rows, k] (k a multiple of 64, at most 1024) into the
  * MFMA-tiled layout [rows rounded up to 16, k]: what dkv_linear's prologue forms,
  * bit for bit, as a launch of its own, whose out is the x of dkv_linear_tiled

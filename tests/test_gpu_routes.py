@@ -233,6 +233,54 @@ def test_long_chunk_without_scratch_for_its_keys(cuda):
         assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize('n,k,q_heads,heads,bits', [
+    (1, 960, 15, 5, 16), (15, 64, 1, 1, 4), (16, 512, 3, 3, 8), (17, 576, 9, 3, 4), (64, 960, 15, 5, 4),
+    (78, 1024, 16, 8, 8), (200, 960, 15, 5, 8), (100, 960, 15, 5, 16),
+])
+@pytest.mark.parametrize('tiled', [False, True])
+def test_projection_that_packs_equals_its_parts(cuda, n, k, q_heads, heads, bits, tiled):
+    """dkv_linear_rope_pack against linear() and append_projection() (themselves checked against torch and
+    the quantizer): q, k, v, the packed bytes and the tile table, bit for bit; one to thirteen row blocks
+    with ragged last ones, one and two pairs of k per wave, behind another segment, with the job in the argument block and in device memory."""
+    import ctypes
+
+    from dkv import _lib
+    announce(f'routes: projection and pack n={n} k={k} heads={q_heads}/{heads} bits={bits} tiled={tiled}')
+    g = torch.Generator().manual_seed(n + k)
+    bf = torch.bfloat16
+    x = (torch.randn(n, k + 8, generator=g) * 2).to(bf).to(cuda)[:, :k]
+    w = (torch.randn((q_heads + 2 * heads) * 64, k, generator=g) / k ** 0.5).to(bf).to(cuda)
+    nw = (torch.rand(k, generator=g) + 0.5).to(bf).to(cuda)
+    angle = torch.rand(n, 64, generator=g) * 6
+    cos, sin = angle.cos().to(bf).to(cuda), angle.sin().to(bf).to(cuda)
+    wt = gpu_ops.mfma_tiled(w) if tiled else None
+    a, b, c = (GPUCache(None, layers=2, heads=heads, max_tokens=n + 9) for _ in range(3))
+    lead = torch.randn(1, heads, 9, 64, generator=g).to(bf).to(cuda)
+    for cache in (a, b, c):
+        cache.arena.zero_()
+        cache.tiles.zero_()
+        cache.select(8, 0)
+        cache.append(lead, lead, 0)
+        cache.select(bits, 1)
+    qkv = gpu_ops.linear(x, w, norm=nw, eps=1e-5, weight_tiled=wt)
+    want = a.append_projection(qkv[None], cos[None], sin[None], q_heads, 0)
+    lib = _lib.load()
+    for cache, on_device in ((b, 0), (c, 1)):
+        past, seg, write_tiles = cache._claim(0, n)
+        q, kn, v = (torch.full_like(t, float('nan')) for t in want[:3])
+        job = cache._job(kn, v, 0, past, n, seg, write_tiles)
+        dev = torch.frombuffer(bytearray(bytes(job)), dtype=torch.uint8).to(cuda)
+        src = w if wt is None else wt
+        _lib.check(lib.dkv_linear_rope_pack(
+            x.data_ptr(), x.stride(0), src.data_ptr(), src.stride(0), n, k, nw.data_ptr(), 1e-5,
+            gpu_ops.LINEAR_W_TILED if tiled else 0, cos.data_ptr(), sin.data_ptr(), 64, q_heads, q.data_ptr(), kn.data_ptr(), v.data_ptr(),
+            dev.data_ptr() if on_device else ctypes.byref(job), on_device, cache.arena.data_ptr(), cache.arena_bytes,
+            cache.tiles.data_ptr(), 2, heads, _lib.stream_handle(cuda)), 'dkv_linear_rope_pack')
+        for got, ref in zip((q, kn, v), want):
+            assert torch.equal(got, ref)
+        assert torch.equal(cache.arena, a.arena) and torch.equal(cache.tiles, a.tiles)
+
+
 @pytest.mark.parametrize('layers,heads,lengths', [
     (3, 5, [64, 64, 64]), (2, 3, [1, 63, 65, 130, 7]), (1, 1, [64] * 128 + [5]), (2, 2, [1] * 300),
     (4, 8, [200]),
