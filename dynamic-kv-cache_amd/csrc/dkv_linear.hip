@@ -423,8 +423,8 @@ __device__ __forceinline__ void lds_operands(uint32_t x, uint32_t w, Op8 (&xa)[2
       : "memory");
 }
 
-template <int EPI, int OPS>
-__global__ void __launch_bounds__(256, 3) linear_tile_kernel(const LinearArgs a) {
+template <int EPI, int OPS, typename Rope>
+__device__ __forceinline__ void tile_body(const LinearArgs& a, const Rope& rope) {
   constexpr int NT = EPI == EPI_SILU_MUL ? TILE_N / 2 : TILE_N;  // output columns of the workgroup
   constexpr int NH = EPI == EPI_SILU_MUL ? 1 : 2;                // 16-column blocks of them per wave
   constexpr int XF = TILE_M / 8, F = XF + TILE_N / 8, FW = F / 4;  // 1 KB pieces of a pair: of x, in all, per wave
@@ -531,6 +531,39 @@ __global__ void __launch_bounds__(256, 3) linear_tile_kernel(const LinearArgs a)
   // The loads past the last pair still write this workgroup's LDS.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
+  if constexpr (EPI == EPI_ROPE) {
+    // A tile is 64 rows of one 64-wide head: rounded to bf16 they meet in LDS (over the operand
+    // buffers, once every wave's last loads have landed), and a wave rotates and packs 16 of them.
+    constexpr int RS = D + 8;  // LDS row, in elements
+    static_assert(TILE_N == D && TILE_M * RS * 2 <= (int)sizeof(lds), "one head per workgroup");
+    uint16_t* head_rows = reinterpret_cast<uint16_t*>(lds);
+    const dkv_pack_job job = rope.djob ? *rope.djob : rope.hjob;
+    const int c = lane & 7;
+    u32x4 cs[2], sn[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int64_t o = (int64_t)min(m0 + 16 * wave + 8 * i + (lane >> 3), a.rows - 1) * rope.cs_stride + 8 * c;
+      cs[i] = *reinterpret_cast<const u32x4*>(rope.cosv + o);
+      sn[i] = *reinterpret_cast<const u32x4*>(rope.sinv + o);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb)
+        *reinterpret_cast<uint2*>(head_rows + (16 * (wm * 2 + mb) + col) * RS + 16 * (wn * 2 + nb) + 4 * g) =
+            make_uint2(pack_bf16(sum[mb][nb][0], sum[mb][nb][1]), pack_bf16(sum[mb][nb][2], sum[mb][nb][3]));
+    __syncthreads();
+    if (ct == 0 && rg == 0 && wave == 0 && job.write_tiles) write_segment_tiles(job, rope.layers, rope.heads, rope.tiles);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int r = 16 * wave + 8 * i + (lane >> 3), tok = m0 + r;
+      rope_pack_row(*reinterpret_cast<const u32x4*>(head_rows + r * RS + 8 * c), cs[i], sn[i], ct, tok, tok < a.rows, c,
+                    a.rows, rope.q_heads, rope.q_out, rope.k_out, rope.v_out, job, rope.arena, rope.layers, rope.heads);
+    }
+    return;
+  }
+
   uint2 resv[2][2];
   if constexpr (EPI == EPI_RESIDUAL) {
 #pragma unroll
@@ -567,6 +600,19 @@ __global__ void __launch_bounds__(256, 3) linear_tile_kernel(const LinearArgs a)
       *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3]));
     }
   }
+}
+
+template <int EPI, int OPS>
+__global__ void __launch_bounds__(256, 3) linear_tile_kernel(const LinearArgs a) {
+  tile_body<EPI, OPS>(a, NoRope{});
+}
+
+// Q/K/V of many rows, ending in dkv_rope_pack's work as linear_rope_kernel does: the 960-wide decoder's
+// launch at 1000 rows 12.6 us instead of 10.4 + 4.3. A whole layer past 640 in graph replays, two launches
+// -> one: 380 rows 64.6 -> 63.4 us, 512 rows 71.1 -> 69.9, 700 rows 77.5 -> 75.5, 1000 rows 81.7 -> 79.0.
+template <int OPS>
+__global__ void __launch_bounds__(256, 3) linear_tile_rope_kernel(const LinearArgs a, const RopeArgs rope) {
+  tile_body<EPI_ROPE, OPS>(a, rope);
 }
 
 // RMSNorm of x rows into the MFMA-tiled layout, for linear_tile_kernel: linear_kernel's prologue as
@@ -803,11 +849,11 @@ int dkv_linear_rope_pack(const void* x, int64_t x_row_stride, const void* w, int
                          const dkv_pack_job* job, int32_t job_on_device, void* arena, int64_t arena_bytes,
                          dkv_tile* tiles, int32_t layers, int32_t heads, void* stream) {
   clear_error();
-  const bool wt = layout & LAYOUT_W_TILED;
-  if (!x || !w || !norm_weight || !cos || !sin || !q_out || !k_out || !v_out || !job || !arena || !tiles || n < 1 ||
-      k <= 0 || (k & 63) || k > 64 * 8 * MAX_NORM_CH || q_heads <= 0 || heads <= 0 || layers <= 0 ||
-      (layout & ~LAYOUT_W_TILED) || !al16(x) || !al16(w) || !al16(norm_weight) || !al16(cos) || !al16(sin) ||
-      !al16(q_out) || !al16(k_out) || !al16(v_out) || (x_row_stride & 7) || x_row_stride < k ||
+  const bool wt = layout & LAYOUT_W_TILED, xt = layout & LAYOUT_X_TILED;
+  if (!x || !w || (norm_weight == nullptr) != xt || !cos || !sin || !q_out || !k_out || !v_out || !job || !arena || !tiles ||
+      n < 1 || k <= 0 || (k & 63) || k > 64 * 8 * MAX_NORM_CH || q_heads <= 0 || heads <= 0 || layers <= 0 ||
+      (layout & ~(LAYOUT_W_TILED | LAYOUT_X_TILED)) || !al16(x) || !al16(w) || !al16(norm_weight) || !al16(cos) ||
+      !al16(sin) || !al16(q_out) || !al16(k_out) || !al16(v_out) || (!xt && ((x_row_stride & 7) || x_row_stride < k)) ||
       (!wt && ((w_row_stride & 7) || w_row_stride < k)) || (cs_row_stride & 7) || cs_row_stride < D) {
     set_error("dkv_linear_rope_pack: bad arguments (%d rows of %d; at least one row, k a multiple of 64 up to %d, 16-byte "
               "aligned bf16 buffers, strides multiples of 8 elements)", n, k, 64 * 8 * MAX_NORM_CH);
@@ -849,9 +895,13 @@ int dkv_linear_rope_pack(const void* x, int64_t x_row_stride, const void* w, int
   r.q_heads = q_heads;
   r.heads = heads;
   r.layers = layers;
-  const dim3 grid((unsigned)((a.n_tiles + 7) / 8) * 8u * (unsigned)a.row_groups);
   hipStream_t st = (hipStream_t)stream;
-  if (a.kp <= 8) {
+  if (xt) a.row_groups = (n + TILE_M - 1) / TILE_M;
+  const dim3 grid((unsigned)((a.n_tiles + 7) / 8) * 8u * (unsigned)a.row_groups);
+  if (xt) {
+    if (wt) hipLaunchKernelGGL((linear_tile_rope_kernel<LAYOUT_X_TILED | LAYOUT_W_TILED>), grid, dim3(256), 0, st, a, r);
+    else hipLaunchKernelGGL((linear_tile_rope_kernel<LAYOUT_X_TILED>), grid, dim3(256), 0, st, a, r);
+  } else if (a.kp <= 8) {
     if (wt) hipLaunchKernelGGL((linear_rope_kernel<1, LAYOUT_W_TILED>), grid, dim3(512), 0, st, a, r);
     else hipLaunchKernelGGL((linear_rope_kernel<1, 0>), grid, dim3(512), 0, st, a, r);
   } else {

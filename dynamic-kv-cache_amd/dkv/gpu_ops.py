@@ -300,8 +300,8 @@ def _layer_plan(layer, n, width):
     # many rows: the norms as launches of their own, before Q/K/V and gate/up
     p.norm1_apart = _prenorm(n, p.qkv_w.shape[0], width, LINEAR_PLAIN)
     p.norm2_apart = _prenorm(n, p.gu_w.shape[0], width, LINEAR_SILU_MUL)
-    # otherwise Q/K/V goes on to RoPE and the pack in its own launch (faster at every such size)
-    p.rope_in_qkv = p.eager_ok and n > 0 and not p.norm1_apart
+    # Q/K/V goes on to RoPE and the pack in its own launch (faster at every size, see the kernels)
+    p.rope_in_qkv = p.eager_ok and n > 0
     plans[(n, width)] = p
     return p
 
@@ -399,7 +399,7 @@ def fused_decoder_layer(layer, hidden_states, cache, position_embeddings):
     x = h.reshape(n, width)
     qt, ot, gt, dt = tiles if tiles is not None else (None,) * 4
     packed = None
-    if p.rope_in_qkv and p.kv_heads == cache.heads and cache._graph is not None:
+    if p.rope_in_qkv and not p.norm1_apart and p.kv_heads == cache.heads and cache._graph is not None:
         cos, sin = position_embeddings
         if (x.stride(-1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and cos.shape == (1, n, 64)
                 and sin.shape == cos.shape and all(t.is_cuda and t.dtype == torch.bfloat16 and t.stride(-1) == 1

@@ -352,7 +352,8 @@ int dkv_linear_tiled(const void* x, int64_t x_row_stride, const void* w, int64_t
 
 /* dkv_linear with the RMSNorm prologue over the joined [q | k | v] weight (k columns, (q_heads + 2 heads) * 64
  * rows), then dkv_rope_pack on the result, in one launch: the same q_out, k_out, v_out and packed bytes. x has n >= 1
- * rows of k (a multiple of 64, at most 1024); layout is 0 or DKV_LINEAR_W_TILED; the rest as those two take it. */
+ * rows of k (a multiple of 64, at most 1024); layout is 0 or DKV_LINEAR_W_TILED; the rest as those two take it.
+ * With DKV_LINEAR_X_TILED x is dkv_rms_norm_tiled's output and norm_weight null (many rows: dkv_linear_prenorm). */
 int dkv_linear_rope_pack(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride, int32_t n, int32_t k,
                          const void* norm_weight, float eps, int32_t layout, const void* cos, const void* sin,
                          int64_t cs_row_stride, int32_t q_heads, void* q_out, void* k_out, void* v_out,
