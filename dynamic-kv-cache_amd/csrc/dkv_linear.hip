@@ -423,6 +423,19 @@ __device__ __forceinline__ void lds_operands(uint32_t x, uint32_t w, Op8 (&xa)[2
       : "memory");
 }
 
+// A pair's eight pieces of x: (step, block of 16 rows).
+__device__ __forceinline__ void lds_pair(uint32_t x, Op8 (&xa)[2][4]) {
+  asm volatile(
+      "ds_read_b128 %0, %8\n ds_read_b128 %1, %8 offset:2048\n"
+      "ds_read_b128 %2, %8 offset:4096\n ds_read_b128 %3, %8 offset:6144\n"
+      "ds_read_b128 %4, %8 offset:1024\n ds_read_b128 %5, %8 offset:3072\n"
+      "ds_read_b128 %6, %8 offset:5120\n ds_read_b128 %7, %8 offset:7168\n s_waitcnt lgkmcnt(0)"
+      : "=&v"(xa[0][0].u), "=&v"(xa[0][1].u), "=&v"(xa[0][2].u), "=&v"(xa[0][3].u), "=&v"(xa[1][0].u),
+        "=&v"(xa[1][1].u), "=&v"(xa[1][2].u), "=&v"(xa[1][3].u)
+      : "v"(x)
+      : "memory");
+}
+
 template <int EPI, int OPS, typename Rope>
 __device__ __forceinline__ void tile_body(const LinearArgs& a, const Rope& rope) {
   constexpr int NT = EPI == EPI_SILU_MUL ? TILE_N / 2 : TILE_N;  // output columns of the workgroup
@@ -615,6 +628,135 @@ __global__ void __launch_bounds__(256, 3) linear_tile_rope_kernel(const LinearAr
   tile_body<EPI_ROPE, OPS>(a, rope);
 }
 
+// SiLU*up over [gate | up] weights for many rows, linear_tile_kernel's arithmetic. A wave owns 64 x rows by
+// 16 gate and 16 up columns, so no weight tile is shared between waves: each goes straight from memory to
+// the registers of the one wave that multiplies it, two pairs ahead, and only x passes through LDS: 24 KB of
+// loads per 64 x 128 weight rows and pair instead of 32, and 40 KB of LDS traffic instead of 96. It needs
+// the chip full, since a workgroup covers twice the columns (GLU_FROM): gate/up of the 960-wide decoder,
+// 64 x 64 tiles -> this, us per launch: 256 rows (160 workgroups) 8.9 -> 9.7, 512 rows (320) 12.0 -> 12.2,
+// 1000 rows (640) 19.6 -> 18.4, 2048 rows (1280) 37.1 -> 30.5. It is bound as the tiles are, by the
+// bytes a CU takes from L2. (A ring of 4 spilled; reading x a step at a time changed nothing.)
+constexpr int GLU_RING = 3;
+constexpr int GLU_N = 64;      // output columns of a workgroup: 4 waves of 16
+constexpr int GLU_FROM = 512;  // workgroups from which it runs (two per CU)
+
+template <int OPS>
+__global__ void __launch_bounds__(256, 3) linear_glu_kernel(const LinearArgs a) {
+  constexpr int XF = TILE_M / 8, XW = XF / 4;  // 1 KB pieces of x per pair, and per wave
+  __shared__ __attribute__((aligned(1024))) u32x4 lds[GLU_RING * XF][64];
+  const int b = blockIdx.x;
+  const int xcd = b & 7, j = b >> 3;
+  const int rg = j % a.row_groups;
+  const int ct = (j / a.row_groups) * 8 + xcd;
+  if (ct >= a.n_tiles) return;  // uniform over the workgroup
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
+  const int n0 = ct * GLU_N + 16 * wave, m0 = rg * TILE_M;
+  const int nl = min(n0, a.up - 16);  // a wave past the last column loads the last columns and stores nothing
+  constexpr bool w_tiled = OPS & LAYOUT_W_TILED, x_tiled = OPS & LAYOUT_X_TILED;
+  constexpr int wsp = w_tiled ? 1024 : 64, wsh = w_tiled ? 512 : 32;
+
+  const uint16_t* xsrc[XW];  // this wave's pieces: block f / 2 of x, MFMA step f % 2
+#pragma unroll
+  for (int q = 0; q < XW; ++q) {  // rows past the end read the last row (block) and are not stored
+    const int f = wave + 4 * q, h = f & 1, row = m0 + 16 * (f >> 1);
+    xsrc[q] = x_tiled ? a.x + (int64_t)min(row >> 4, (a.rows - 1) >> 4) * a.kp * 1024 + 512 * h + 8 * lane
+                      : a.x + (int64_t)min(row + col, a.rows - 1) * a.ldx + 32 * h + 8 * g;
+  }
+  const uint16_t* wsrc[2];  // gate, up
+#pragma unroll
+  for (int nb = 0; nb < 2; ++nb) {
+    const int r = nl + nb * a.up;
+    wsrc[nb] = w_tiled ? a.w + (int64_t)(r >> 4) * a.kp * 1024 + 8 * lane : a.w + (int64_t)(r + col) * a.ldw + 8 * g;
+  }
+  auto next = [&](int p) {  // the pair after p: the next of its chain, or the next chain's first
+    const int q = p + 8;
+    return q < a.kp ? q : (p & 7) + 1;
+  };
+  // Past the last pair the last one is loaded again (never used), so that every pair has as many loads
+  // after it.
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
+  Op8 w[GLU_RING][2][2];
+  int pl = 0, loaded = 0, fill = 0;  // pair loaded next, its place in the order, its buffer
+  auto load_next = [&](Op8 (&to)[2][2]) {
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) to[nb][h].u = *reinterpret_cast<const u32x4*>(wsrc[nb] + wsp * pl + wsh * h);
+#pragma unroll
+    for (int q = 0; q < XW; ++q)
+      asm volatile("s_mov_b32 m0, %1\n s_nop 0\n global_load_lds_dwordx4 %0, off" ::"v"(xsrc[q] + (x_tiled ? 1024 : 64) * pl),
+                   "s"(lds0 + 1024 * (fill * XF + wave + 4 * q)) : "memory");
+    fill = fill + 1 == GLU_RING ? 0 : fill + 1;
+    if (++loaded < a.kp) pl = next(pl);
+  };
+  f32x4_t acc[4][2], sum[4][2];  // the chain in progress; the chains done
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) {
+      acc[mb][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      sum[mb][nb] = f32x4_t{-0.f, -0.f, -0.f, -0.f};  // -0 + x is x, for every x
+    }
+  const uint32_t base = lds0 + 16 * lane;
+#pragma unroll
+  for (int k = 0; k < GLU_RING - 1; ++k) load_next(w[k]);
+  int p = 0;  // pair being computed
+  for (int s0 = 0; s0 < a.kp; s0 += GLU_RING) {
+#pragma unroll
+    for (int i = 0; i < GLU_RING; ++i) {  // pair s0 + i, in buffer i
+      if (s0 + i >= a.kp) break;
+      // The pair's pieces have landed (this wave's: only the GLU_RING - 2 pairs after it are under way;
+      // the other waves': the barrier), and every wave is past the pair before it.
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((GLU_RING - 2) * (XW + 4)) : "memory");
+      // the wait above is for this pair's weights too; the compiler places its own here, not after the
+      // loads below
+      asm volatile("" : "+v"(w[i][0][0].u), "+v"(w[i][0][1].u), "+v"(w[i][1][0].u), "+v"(w[i][1][1].u));
+      __builtin_amdgcn_s_barrier();
+      load_next(w[(i + GLU_RING - 1) % GLU_RING]);
+      const uint32_t at = base + 1024 * XF * i;
+      Op8 xa[2][4];
+      lds_pair(at, xa);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+          for (int nb = 0; nb < 2; ++nb)
+            acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i][nb][h].v, xa[h][mb].v, acc[mb][nb], 0, 0, 0);
+      if (p + 8 >= a.kp) {  // the chain's last pair
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+          for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              sum[mb][nb][e] += acc[mb][nb][e];
+              acc[mb][nb][e] = 0.f;
+            }
+      }
+      p = next(p);
+    }
+  }
+  // The loads past the last pair still write this workgroup's LDS.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (n0 >= a.up) return;
+  const int c = n0 + 4 * g;
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb) {
+    const int row = m0 + 16 * mb + col;
+    if (row >= a.rows) continue;
+    float y[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float x = round_bf16(sum[mb][0][e]);
+      y[e] = round_bf16(x / (1.f + expf(-x))) * round_bf16(sum[mb][1][e]);
+    }
+    uint16_t* dst = a.out + ((a.layout & LAYOUT_OUT_TILED) ? tiled_offset(row, c, a.up >> 6) : (int64_t)row * a.ldo + c);
+    *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3]));
+  }
+}
+
 // RMSNorm of x rows into the MFMA-tiled layout, for linear_tile_kernel: linear_kernel's prologue as
 // a launch of its own (there every workgroup normalizes its x rows again; with 16 times the rows per
 // weight tile that work is worth doing once). One workgroup per 16 rows; wave w sums and normalizes
@@ -730,7 +872,16 @@ void launch_one(const LinearArgs& a, hipStream_t st) {
 }
 
 template <int EPI, int OPS>
-void launch_tile(const LinearArgs& a, hipStream_t st) {
+void launch_tile(LinearArgs a, hipStream_t st) {
+  if constexpr (EPI == EPI_SILU_MUL) {
+    const int wide = (a.up + GLU_N - 1) / GLU_N;
+    if ((int64_t)wide * a.row_groups >= GLU_FROM) {
+      a.n_tiles = wide;
+      hipLaunchKernelGGL((linear_glu_kernel<OPS>), dim3((unsigned)((wide + 7) / 8) * 8u * (unsigned)a.row_groups), dim3(256), 0,
+                         st, a);
+      return;
+    }
+  }
   const unsigned blocks = (unsigned)((a.n_tiles + 7) / 8) * 8u * (unsigned)a.row_groups;
   hipLaunchKernelGGL((linear_tile_kernel<EPI, OPS>), dim3(blocks), dim3(256), 0, st, a);
 }

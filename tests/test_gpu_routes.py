@@ -59,6 +59,7 @@ def test_attend_calls_share_no_workspace(cuda):
     (700, 512, 448, False, 'plain'), (4500, 576, 64, True, 'plain'), (321, 960, 960, False, 'residual'),
     (385, 960, 1600, True, 'plain'), (97, 960, 5120, True, 'silu'), (130, 960, 5120, False, 'silu'),
     (2071, 1024, 256, True, 'silu'),
+    (1000, 960, 5120, True, 'silu'), (2049, 512, 2112, False, 'silu'), (8200, 64, 576, False, 'silu'), (577, 2560, 960, False, 'residual'), (3000, 2560, 192, False, 'plain'),
 ])
 def test_many_row_projections_equal_few_row_ones(cuda, rows, k, n, norm, epi):
     """From some hundred rows on linear() runs 64 x 64 tiles (and the norm as a launch of its own).
