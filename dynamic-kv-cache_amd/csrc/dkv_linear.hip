@@ -634,7 +634,7 @@ __global__ void __launch_bounds__(256, 3) linear_tile_rope_kernel(const LinearAr
 // loads per 64 x 128 weight rows and pair instead of 32, and 40 KB of LDS traffic instead of 96. It needs
 // the chip full, since a workgroup covers twice the columns (GLU_FROM): gate/up of the 960-wide decoder,
 // 64 x 64 tiles -> this, us per launch: 256 rows (160 workgroups) 8.9 -> 9.7, 512 rows (320) 12.0 -> 12.2,
-// 1000 rows (640) 19.6 -> 18.4, 2048 rows (1280) 37.1 -> 30.5. It is bound as the tiles are, by the
+// 1000 rows (640) 19.6 -> 17.6, 2048 rows (1280) 37.1 -> 28.8. It is bound as the tiles are, by the
 // bytes a CU takes from L2. (A ring of 4 spilled; reading x a step at a time changed nothing.)
 constexpr int GLU_RING = 3;
 constexpr int GLU_N = 64;      // output columns of a workgroup: 4 waves of 16

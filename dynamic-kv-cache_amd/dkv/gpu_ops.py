@@ -10,9 +10,9 @@ patched attention forward in one launch (dkv_rope_qkv).
 linear() is libdkv's short-chunk projection (dkv_linear): the joined GEMMs on
 MFMA with the RMSNorm before them and the residual add or SiLU*up after them
 folded in. install_fused_ops also patches LlamaDecoderLayer so that, on a
-packed GPUCache, a layer runs as five launches plus the attention: Q/K/V
-(with input_layernorm), split + RoPE + pack, attention, o_proj + residual,
-gate/up (with post_attention_layernorm) + SiLU*up, down_proj + residual.
+packed GPUCache, a layer runs as four launches plus the attention: Q/K/V (with
+input_layernorm before and split + RoPE + pack after), o_proj +
+residual, gate/up (with post_attention_layernorm) + SiLU*up, down_proj + residual.
 
 Tensors the kernels do not cover (other dtypes, CPU tensors, other shapes)
 take the reference's own torch composition.
