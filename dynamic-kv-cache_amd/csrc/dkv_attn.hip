@@ -520,6 +520,10 @@ static bool prompt_route(const dkv_attn_args& a) {
          (int64_t)(a.q_heads / a.heads) * a.nq >= PROMPT_ROWS;
 }
 
+static PromptPlan make_prompt_plan(const dkv_attn_args& a) {
+  return prompt_plan(a, num_cus(), a.precision == 0 && make_plan(a).splits > 1);
+}
+
 // Workspace bytes of a plan: the split partials (none for one split), after the arrival counters in
 // the in-kernel merge build.
 static int64_t workspace_bytes(const Plan& p) {
@@ -625,7 +629,7 @@ extern "C" {
 int64_t dkv_attend_workspace_bytes(const dkv_attn_args* args) {
   if (!args || args->heads <= 0 || args->q_heads <= 0 || args->q_heads % args->heads || args->nq <= 0)
     return 0;
-  return prompt_route(*args) ? prompt_plan(*args, num_cus()).bytes() : workspace_bytes(make_plan(*args));
+  return prompt_route(*args) ? make_prompt_plan(*args).bytes() : workspace_bytes(make_plan(*args));
 }
 
 int dkv_attend(const dkv_attn_args* args, void* stream) {
@@ -639,7 +643,7 @@ int dkv_attend(const dkv_attn_args* args, void* stream) {
   const bool prompt = prompt_route(a);
   PromptPlan pp;
   Plan p;
-  if (prompt) pp = prompt_plan(a, num_cus());
+  if (prompt) pp = make_prompt_plan(a);
   else p = make_plan(a);
   const int64_t need = prompt ? pp.bytes() : workspace_bytes(p);
   if (need > 0 && (!a.workspace || a.workspace_bytes < need)) {
@@ -661,7 +665,7 @@ int dkv_attend_noalloc(const dkv_attn_args* args, void* stream) {
   if (int rc = check_args(a)) return rc;
   if (prompt_route(a)) {
     // (a chunk whose unpacked keys and partials pass the scratch buffer runs the frame-chunk plan)
-    const PromptPlan pp = prompt_plan(a, num_cus());
+    const PromptPlan pp = make_prompt_plan(a);
     if (pp.bytes() <= DKV_NOALLOC_SCRATCH_BYTES) {
       void* ws = nullptr;
       if (int rc = scratch_address(&ws)) return rc;

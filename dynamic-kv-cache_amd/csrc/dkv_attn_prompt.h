@@ -33,11 +33,17 @@ __host__ __device__ inline int prompt_splits(int units, int unit_len) { return (
 struct PromptPlan {
   int groups, units, unit_len, max_splits;
   int ranges;  // of one KV head, over all groups
+  // Partials of groups with several ranges as fp16 O / sum (half_slot() order) rather than fp32 O: only
+  // where the frame-chunk plan of the same call stores fp16 partials too. Longer chunks (about 24600 query
+  // rows over all Q heads, 256 CUs) run one split there, whose O stays in fp32, and keep it so here; fp16
+  // would take 2048 tokens past 1000 from 45.3 to 43.4 us and 8192 tokens from 186 to 180 (15 Q / 5 KV
+  // heads, bf16) at an error against float64 of 2.682e-3 instead of 2.677e-3.
+  bool half;
   int64_t image_bytes, part_o_bytes, part_ml_bytes;
   int64_t bytes() const { return image_bytes + part_o_bytes + part_ml_bytes; }
 };
 
-PromptPlan prompt_plan(const dkv_attn_args& a, int cus);
+PromptPlan prompt_plan(const dkv_attn_args& a, int cus, bool half);
 // ws: PromptPlan::bytes() bytes, 16-byte aligned.
 int launch_attn_prompt(const dkv_attn_args& a, const PromptPlan& p, void* ws, hipStream_t s);
 

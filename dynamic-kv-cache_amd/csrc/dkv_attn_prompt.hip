@@ -19,11 +19,11 @@
 // What bounds it: the softmax's VALU work (about 130 instructions and 32 exponentials per wave and
 // unit beside 32 MFMAs), then the two small launches around it (4 to 5 us each). Frame-chunk kernel ->
 // these, us per call, 15 Q / 5 KV heads, bf16 (fp32 precision):
-//    512 tokens past 1024   22.2 ->  18.6   (28.0 -> 23.5)
-//   1000 tokens past  640   36.1 ->  21.9   (45.5 -> 29.3)
-//   2048 tokens past 1000   88.9 ->  41.2  (105.3 -> 61.2)
-//   2048 tokens past 8128  266.5 -> 101.8  (342.1 -> 190.4)
-//   8192 tokens            652.9 -> 178.9  (782.8 -> 281.0)   720 TFLOP/s of causal work
+//    512 tokens past 1024   23.7 ->  19.6   (29.1 -> 24.6)
+//   1000 tokens past  640   36.8 ->  22.8   (46.0 -> 30.7)
+//   2048 tokens past 1000   88.5 ->  45.3  (104.5 -> 65.1)
+//   2048 tokens past 8128  266.5 -> 113.0  (338.6 -> 190.5)
+//   8192 tokens            648.0 -> 187.0  (785.0 -> 286.0)   690 TFLOP/s of causal work
 // Precision 0 rounds K, V and p to bf16, precision 1 splits each in two bf16 parts, as the
 // frame-chunk kernel does (dkv_attn_mfma.hip).
 #include "dkv_attn_common.h"
@@ -246,7 +246,8 @@ __device__ __forceinline__ void load_piece(const uint8_t* from, uint32_t to) {
   asm volatile("s_mov_b32 m0, %1\n s_nop 0\n global_load_lds_dwordx4 %0, off" ::"v"(from), "s"(to) : "memory");
 }
 
-template <int PREC>
+// HALF: the partials of groups with several ranges, see PromptPlan::half.
+template <int PREC, bool HALF>
 __global__ void __launch_bounds__(64 * PROMPT_WAVES, 4)
 prompt_kernel(dkv_attn_args a, int units, int unit_len, int max_splits, int groups, const uint8_t* __restrict__ images,
               float* __restrict__ part_o, float2* __restrict__ part_ml) {
@@ -467,7 +468,7 @@ prompt_kernel(dkv_attn_args a, int units, int unit_len, int max_splits, int grou
     }
     const int64_t row = ((int64_t)h * max_splits + split) * ((int64_t)groups * PROMPT_ROWS) + grp * PROMPT_ROWS +
                         32 * wave + lr;
-    if (PREC) {
+    if (!HALF) {
 #pragma unroll
       for (int db = 0; db < 4; ++db)
         __builtin_nontemporal_store(acc[nb][db], reinterpret_cast<pf32x4*>(part_o + row * D + 16 * db + 4 * g));
@@ -506,11 +507,11 @@ prompt_kernel(dkv_attn_args a, int units, int unit_len, int max_splits, int grou
 // 3. The merge. A lane holds one 16-byte chunk of one row and walks the row's splits, four loads at a
 // time: no exchange between lanes. (The frame-chunk merge spreads a row's splits, up to 51, over the
 // lanes of a wave; here a row has two to about ten.)
-template <int PREC>
+template <bool HALF>
 __global__ void __launch_bounds__(256)
 prompt_merge_kernel(dkv_attn_args a, int unit_len, int max_splits, int groups, const float* __restrict__ part_o,
                     const float2* __restrict__ part_ml) {
-  constexpr int CH = PREC ? 16 : 8;  // 16-byte chunks per row
+  constexpr int CH = HALF ? 8 : 16;  // 16-byte chunks per row
   const int h = blockIdx.y;
   const int64_t rows = (int64_t)groups * PROMPT_ROWS;
   const int64_t rp = ((int64_t)blockIdx.x * 256 + threadIdx.x) / CH;
@@ -526,7 +527,7 @@ prompt_merge_kernel(dkv_attn_args a, int unit_len, int max_splits, int groups, c
   const u32x4* po = reinterpret_cast<const u32x4*>(part_o);
   const pf32x2* pml = reinterpret_cast<const pf32x2*>(part_ml);
   const int64_t first = (int64_t)h * max_splits * rows + rp;
-  constexpr int V = PREC ? 4 : 8;
+  constexpr int V = HALF ? 8 : 4;
   float M = -INFINITY, L = 0.f, o[V];
 #pragma unroll
   for (int e = 0; e < V; ++e) o[e] = 0.f;
@@ -552,7 +553,7 @@ prompt_merge_kernel(dkv_attn_args a, int unit_len, int max_splits, int groups, c
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       float w = ml[i][0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[i][0] - bm);
-      if constexpr (PREC) {
+      if constexpr (!HALF) {
         L = fmaf(ml[i][1], w, L);
         const float4 v = __builtin_bit_cast(float4, raw[i]);
         o[0] = fmaf(v.x, w, o[0]);
@@ -577,7 +578,7 @@ prompt_merge_kernel(dkv_attn_args a, int unit_len, int max_splits, int groups, c
   const int64_t off = (int64_t)m * a.out_tok_stride + (int64_t)(h * G + gq) * a.out_head_stride;
 #pragma unroll
   for (int k = 0; k < V / 4; ++k) {
-    const int at = PREC ? 4 * c : half_column(8 * c + 4 * k);
+    const int at = HALF ? half_column(8 * c + 4 * k) : 4 * c;
     const pf32x4 v = {o[4 * k] * inv, o[4 * k + 1] * inv, o[4 * k + 2] * inv, o[4 * k + 3] * inv};
     if (a.out_dtype == 1) *reinterpret_cast<pf32x4*>(static_cast<float*>(a.out) + off + at) = v;
     else *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.out) + off + at) = make_uint2(pk2(v[0], v[1]), pk2(v[2], v[3]));
@@ -587,8 +588,9 @@ prompt_merge_kernel(dkv_attn_args a, int unit_len, int max_splits, int groups, c
 // ---------------------------------------------------------------------------
 // Host side.
 
-PromptPlan prompt_plan(const dkv_attn_args& a, int cus) {
+PromptPlan prompt_plan(const dkv_attn_args& a, int cus, bool half) {
   PromptPlan p;
+  p.half = half;
   const int G = a.q_heads / a.heads;
   p.groups = prompt_groups(G, a.nq);
   p.units = (int)(((int64_t)a.past + a.nq + TILE - 1) / TILE);
@@ -610,28 +612,30 @@ PromptPlan prompt_plan(const dkv_attn_args& a, int cus) {
   p.max_splits = prompt_splits(prompt_group_units(p.groups - 1, G, a.nq, a.past), p.unit_len);
   p.image_bytes = (int64_t)a.heads * p.units * prompt_image_bytes(a.precision);
   const int64_t rows = p.max_splits > 1 ? (int64_t)a.heads * p.max_splits * p.groups * PROMPT_ROWS : 0;
-  p.part_o_bytes = rows * D * (a.precision ? 4 : 2);
+  p.part_o_bytes = rows * D * (half ? 2 : 4);
   p.part_ml_bytes = rows * 8;
   return p;
 }
 
-template <int PREC>
+template <int PREC, bool HALF>
 static void launch_prec(const dkv_attn_args& a, const PromptPlan& p, uint8_t* ws, hipStream_t s) {
   float* part_o = reinterpret_cast<float*>(ws + p.image_bytes);
   float2* part_ml = reinterpret_cast<float2*>(ws + p.image_bytes + p.part_o_bytes);
   hipLaunchKernelGGL(prompt_tiles_kernel<PREC>, dim3(p.units, a.heads), dim3(256), 0, s, a, ws);
-  hipLaunchKernelGGL(prompt_kernel<PREC>, dim3(p.ranges * a.heads), dim3(64 * PROMPT_WAVES), 0, s, a, p.units,
+  hipLaunchKernelGGL((prompt_kernel<PREC, HALF>), dim3(p.ranges * a.heads), dim3(64 * PROMPT_WAVES), 0, s, a, p.units,
                      p.unit_len, p.max_splits, p.groups, ws, part_o, part_ml);
   if (p.max_splits > 1) {
-    const int64_t threads = (int64_t)p.groups * PROMPT_ROWS * (PREC ? 16 : 8);
-    hipLaunchKernelGGL(prompt_merge_kernel<PREC>, dim3((unsigned)(threads / 256), a.heads), dim3(256), 0, s, a,
+    const int64_t threads = (int64_t)p.groups * PROMPT_ROWS * (HALF ? 8 : 16);
+    hipLaunchKernelGGL(prompt_merge_kernel<HALF>, dim3((unsigned)(threads / 256), a.heads), dim3(256), 0, s, a,
                        p.unit_len, p.max_splits, p.groups, part_o, part_ml);
   }
 }
 
 int launch_attn_prompt(const dkv_attn_args& a, const PromptPlan& p, void* ws, hipStream_t s) {
-  if (a.precision == 1) launch_prec<1>(a, p, static_cast<uint8_t*>(ws), s);
-  else launch_prec<0>(a, p, static_cast<uint8_t*>(ws), s);
+  uint8_t* w = static_cast<uint8_t*>(ws);
+  if (a.precision == 1) launch_prec<1, false>(a, p, w, s);
+  else if (p.half) launch_prec<0, true>(a, p, w, s);
+  else launch_prec<0, false>(a, p, w, s);
   return (int)hipGetLastError();
 }
 

@@ -197,6 +197,26 @@ def test_decode_workgroups_of_several_units(cuda, heads, group, nq, past, tiles)
         assert bool(((got[0].double() - ref).abs() <= bound).all()), splits
 
 
+@pytest.mark.parametrize('heads,group,nq,past', [(5, 3, 2048, 1000), (2, 8, 1601, 130), (8, 4, 900, 500)])
+def test_long_chunk_sums_stay_in_32_bits(cuda, heads, group, nq, past):
+    """Chunks so long that the frame-chunk kernel runs one history split keep O in fp32 to the end, so
+    the long-chunk kernels' partials must too. With K = 0 every p is 1 and with small whole numbers as V
+    every sum is exact, so an fp32 output is off by the reciprocal and one product: 2^-22 of it (fp16
+    partials: 2^-12)."""
+    announce(f'routes: long chunk sums heads={heads} group={group} nq={nq} past={past}')
+    g = torch.Generator().manual_seed(nq)
+    c = GPUCache(None, layers=1, heads=heads, max_tokens=past + nq)
+    hist = torch.randint(-8, 9, (1, heads, past, 64), generator=g).to(torch.bfloat16).to(cuda)
+    c.append_batch(torch.zeros_like(hist), hist, [16] * ((past + 63) // 64), [min(64, past - t) for t in range(0, past, 64)])
+    q = torch.randn((1, heads * group, nq, 64), generator=g).to(torch.bfloat16).to(cuda)
+    v = torch.randint(-8, 9, (1, heads, nq, 64), generator=g).to(torch.bfloat16).to(cuda)
+    got = c.attend(q, torch.zeros_like(v), v, 0, past, out_dtype=torch.float32)[0].double()
+    seen = torch.arange(past + 1, past + nq + 1, device=cuda, dtype=torch.float64)[:, None, None]
+    ref = ((hist[0].double().sum(1, keepdim=True) + v[0].double().cumsum(1)).transpose(0, 1) / seen)
+    ref = ref.repeat_interleave(group, 1)
+    assert bool(((got - ref).abs() <= 2.0 ** -22 * ref.abs()).all())
+
+
 def test_long_chunk_partials_keep_large_values(cuda):
     """|V| near the top of bf16: the fp16 partial outputs are stored scaled; V and V * 2^20 give outputs
     that differ by exactly that factor, up to the one bit a scaled sum may lose (2^-15)."""
