@@ -31,6 +31,7 @@ BITS = (4, 8, 16)
 PRECISIONS = {'bf16': 0, 'fp32': 1}
 PATHS = {'auto': 0, 'vector': 1, 'mfma': 2, 'short': 3}
 _ONE_SEGMENT = (0,) * (_lib.DKV_MAX_CHUNK_SEGS + 1)  # dkv_attn_args.seg_bounds of an unsegmented chunk
+SMALL_ROWS = 32  # query rows per KV head up to which 'auto' runs the decode-step variant (MFMA_SMALL_ROWS there)
 SHORT_ROWS = 16  # query rows per KV head the short-chunk kernel takes (SHORT_ROWS of csrc/dkv_attn_common.h)
 
 
@@ -116,6 +117,9 @@ class GPUCache(_CacheBase):
         # default `splits` of attend() for chunks of more than SHORT_ROWS query rows per KV head
         # (0: the library's plan, the shortest latency of a launch that has the GPU to itself)
         self.chunk_splits = 0
+        # attend() calls of path 'auto' take the kernels graph replays take: long chunks run the
+        # frame-chunk kernel, as launches with a step pair do (forwards that also run as replays)
+        self.as_replayed = False
         self.online = plan is None
         self.plan = []  # (start, end, bits, row) per segment, as in the reference
         self.segments = []
@@ -442,8 +446,10 @@ class GPUCache(_CacheBase):
         a.arena, a.tiles, a.tiles_host = self.arena.data_ptr(), self.tiles.data_ptr(), self._tiles_host_ptr
         a.n_tiles, a.past, a.layer = self._tiles_before(past), past, layer
         a.precision = PRECISIONS[self.precision]
-        if q_heads // H * n > SHORT_ROWS:
+        rows = q_heads // H * n
+        if rows > SHORT_ROWS:
             a.splits = self.chunk_splits
+        a.path = PATHS['mfma'] if self.as_replayed and rows > SMALL_ROWS else 0
         need = lib.dkv_attend_workspace_bytes(ctypes.byref(a))
         if need:
             ws = self._workspace_for(need)
@@ -561,6 +567,8 @@ class GPUCache(_CacheBase):
         if len(shape) != 4 or shape[0] != 1 or shape[3] != d or shape[1] % heads:
             raise ValueError('attend expects q [1, q_heads, n, 64] with q_heads a multiple of heads')
         _, q_heads, n, _ = shape
+        if path == 0 and self.as_replayed and q_heads // heads * n > SMALL_ROWS:
+            path = PATHS['mfma']
         if k.shape != (1, heads, n, d) or v.shape != k.shape:
             raise ValueError(f'attend expects the chunk k, v of shape [1, {heads}, {n}, {d}]')
         if past + n > self.capacity or past > self.seen[layer]:
@@ -683,6 +691,8 @@ class GPUCache(_CacheBase):
         memory, so that a decoder forward over `chunk`-token chunks can be captured once in a HIP
         graph and replayed as the history grows. Before capturing, and before every replay, call
         graph_step(); in this mode append() and attend() only launch (no bookkeeping).
+        A replay gives the bits of ordinary calls on the same history with `as_replayed` set; without
+        it long chunks run other kernels (attend(), path 'auto'), equal within rounding.
 
         `q_heads` pre-sizes the steps' attention workspace for the launch bounds (so nothing is
         allocated while capturing); graph launches use that buffer, never the one ordinary calls

@@ -95,15 +95,23 @@ class StreamingDecoder:
 
     @torch.inference_mode()
     def forward(self, cache, ids=None, embeddings=None, positions=None, logits=0):
-        """One decoder forward of a chunk. Returns fp32 logits of the last `logits` positions."""
+        """One decoder forward of a chunk. Returns fp32 logits of the last `logits` positions.
+
+        With graphs=True a chunk may run here once and as graph replays later, so its attention runs
+        the kernels that replays run (GPUCache.as_replayed): the outputs are the same bits either way.
+        """
         if embeddings is None:
             embeddings = self.text.get_input_embeddings()(ids.to(self.device))
         past = cache.get_seq_length()
         n = embeddings.shape[1]
         if positions is None:
             positions = torch.arange(past, past + n, device=self.device)
-        out = self.text(inputs_embeds=embeddings, past_key_values=cache, use_cache=True,
-                        position_ids=positions[None], attention_mask=None, return_dict=True)
+        before, cache.as_replayed = getattr(cache, 'as_replayed', False), True
+        try:
+            out = self.text(inputs_embeds=embeddings, past_key_values=cache, use_cache=True,
+                            position_ids=positions[None], attention_mask=None, return_dict=True)
+        finally:
+            cache.as_replayed = before
         if not logits:
             return None
         return self.model.lm_head(out.last_hidden_state[:, -int(logits):]).float()

@@ -101,7 +101,10 @@ typedef struct dkv_attn_args {
   const int32_t* step;   /* NULL, or a DEVICE pair {past, n_tiles} read when the kernels run,
                             for launches recorded once in a HIP graph and replayed as the
                             history grows. `past` and `n_tiles` above then bound the launch
-                            (grid, workspace) and the device pair must stay within them. */
+                            (grid, workspace) and the device pair must stay within them. Such a
+                            launch runs the frame-chunk kernel at every size: bit for bit what path 2
+                            gives without `step`, and what path 0 gives up to long chunks (see
+                            dkv_attend), whose results there are equal within rounding. */
   const dkv_tile* tiles_host; /* NULL, or a HOST copy of tiles[0, n_tiles), equal to the device
                             table. For a launch without `step` and n_tiles <= DKV_ARG_TILES the
                             frame-chunk kernel then takes the descriptors from its argument block

@@ -234,6 +234,50 @@ def test_long_chunk_partials_keep_large_values(cuda):
     assert (a - b).abs().max() <= 2.0 ** -10 * a.abs().max()
 
 
+@pytest.mark.parametrize('precision', ['fp32', 'bf16'])
+@pytest.mark.parametrize('past,nq', [(0, 500), (700, 420)])
+def test_long_chunk_replays_equal_calls_as_replayed(cuda, past, nq, precision):
+    """A long chunk recorded with graph steps runs the frame-chunk kernel: bit for bit what ordinary calls
+    give with as_replayed set or path='mfma', over every replay. The default call differs by rounding: p to bf16 twice, 2^-8 of each term at most
+    and random over rows of hundreds of keys, so under 1% of the outputs' norm."""
+    announce(f'routes: long chunk replay past={past} nq={nq} {precision}')
+    case = frame_chunk_case(max(past, 64), seed=nq, nq=nq)
+    g = torch.Generator().manual_seed(nq)
+    chunks = [[torch.randn((1, h, nq, 64), generator=g).to(torch.bfloat16).to(cuda) for h in (15, 5, 5)] for _ in range(3)]
+
+    def cache():
+        if past:
+            return filled(case, cuda, 5, extra=3 * nq, precision=precision)[0]
+        return GPUCache(None, layers=1, heads=5, max_tokens=3 * nq, precision=precision)
+
+    plain, c = cache(), cache()
+    c.select(8, 1)
+    plain.select(8, 1)
+    steps = c.begin_graph_steps(nq, q_heads=15)
+    past0 = c.graph_step()
+    static = [t.clone() for t in chunks[0]]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        c.append(static[1], static[2], 0)
+        out = c.attend(static[0], static[1], static[2], 0, past0)
+    steps.upload()
+    for i, (q, k, v) in enumerate(chunks):
+        if i:
+            c.graph_step()
+            for dst, src in zip(static, (q, k, v)):
+                dst.copy_(src)
+        graph.replay()
+        at = plain.append(k, v, 0)
+        auto = plain.attend(q, k, v, 0, at)
+        assert torch.equal(out, plain.attend(q, k, v, 0, at, path='mfma'))
+        plain.as_replayed = True
+        assert torch.equal(out, plain.attend(q, k, v, 0, at))
+        plain.as_replayed = False
+        assert (out.float() - auto.float()).norm() <= 0.01 * out.float().norm()
+    c.end_graph_steps()
+
+
 def test_long_chunk_without_scratch_for_its_keys(cuda):
     """dkv_attend_noalloc: the same call as dkv_attend where the unpacked keys and partials fit its
     scratch buffer; where they do not, the frame-chunk kernel's output instead of a refusal."""

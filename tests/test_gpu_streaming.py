@@ -208,6 +208,37 @@ def test_graph_replayed_answers_match_eager(cuda):
     dec.graphs = False
 
 
+@pytest.mark.parametrize('precision', ['fp32', 'bf16'])
+def test_graph_replayed_long_chunks_match_eager(cuda, precision):
+    """A prefix, a frame, a question and a candidate batch of more than a thousand tokens: attend() alone
+    would run them on the long-chunk kernels, which graph replays do not. First requests run them
+    eagerly, later ones as replays, and a decoder without graphs always eagerly: logits, scores and cache
+    bytes must not depend on which."""
+    announce(f'streaming: long chunks, eager vs replays, precision={precision}')
+    model = build_decoder(**dict(SMALL, max_positions=8192), seed=51)
+    dec = StreamingDecoder(model, precision=precision, pipeline=1)
+    g = torch.Generator().manual_seed(52)
+    prefix = torch.randint(0, 512, (1, 1201), generator=g)
+    question = torch.randint(0, 512, (1, 1150), generator=g)
+    cands = [torch.randint(0, 512, (1, n), generator=g) for n in (700, 501)]
+    frames = frames_for(model, 2, seed=53, tokens=1200)
+
+    def request():
+        cache = dec.ingest(prefix, frames, [4, 8], qa_reserve=3000)
+        out = (dec.answer_batched(cache, question, cands),
+               dec.forward(cache.fork(), ids=question, logits=question.shape[1]), *cache.materialize(1))
+        torch.cuda.synchronize()
+        return out
+
+    eager = request()
+    dec.graphs = True
+    for i in range(3):
+        for a, b in zip(request(), eager):
+            assert torch.equal(a, b), (i, (a.float() - b.float()).abs().max().item())
+    assert len(dec._qa_graphs) == 2
+    dec.graphs = False
+
+
 def test_label_protocol_and_calibration_prior(cuda):
     """The 'label' protocol reads the last position's logits at the label ids on a fork (the base
     cache keeps its length), and the calibration prior is the candidate scoring on a prefix-only
