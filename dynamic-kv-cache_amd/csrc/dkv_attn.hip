@@ -356,6 +356,12 @@ static int num_cus() {
   return cus;
 }
 
+// Whether t is a well-formed descriptor of the tile that starts at token `start`.
+static bool tile_at(const dkv_tile& t, int64_t start) {
+  return (t.bits == 4 || t.bits == 8 || t.bits == 16) && t.rows >= 1 && t.rows <= TILE && t.offset >= 0 &&
+         t.token_start == start;
+}
+
 static int check_args(const dkv_attn_args& a) {
   if (!a.q || !a.k_new || !a.v_new || !a.out || (a.n_tiles > 0 && (!a.tiles || !a.arena))) {
     set_error("dkv_attend: null pointer argument");
@@ -412,8 +418,7 @@ static int check_args(const dkv_attn_args& a) {
     int next = 0;
     for (int i = 0; i < a.n_tiles; ++i) {
       const dkv_tile& t = a.tiles_host[i];
-      if ((t.bits != 4 && t.bits != 8 && t.bits != 16) || t.rows < 1 || t.rows > TILE || t.offset < 0 ||
-          t.token_start != next) {
+      if (!tile_at(t, next)) {
         set_error("dkv_attend: tiles_host[%d] (token_start %d, rows %d, bits %d) is not the tile after "
                   "token %d", i, t.token_start, (int)t.rows, (int)t.bits, next);
         return DKV_EINVAL;
@@ -515,9 +520,22 @@ static Plan make_plan(const dkv_attn_args& a) {
 //   16 / 8 heads  4096 rows (256 past 1024) 16.5 -> 17.3   8192 (512 past 1024) 24.0 -> 18.4
 //    9 / 3 heads  2880 rows (320 past 1024) 15.1 -> 16.2   4608 (512 past 1024) 18.1 -> 16.8
 static constexpr int64_t PROMPT_FROM = 4500;
+// These kernels look every history token up in the tile table, where the frame-chunk kernel walks the
+// tiles there are and clamps each to its rows: they run only where the host copy of the table shows a tile
+// for each token below past (well under 1 ns per tile and call).
+static bool table_covers(const dkv_attn_args& a) {
+  if (a.past <= 0) return true;
+  if (!a.tiles_host) return false;
+  int64_t next = 0;
+  for (int i = 0; i < a.n_tiles; ++i) {
+    if (!tile_at(a.tiles_host[i], next)) return false;
+    next += a.tiles_host[i].rows;
+  }
+  return next >= a.past;
+}
 static bool prompt_route(const dkv_attn_args& a) {
   return a.path == 0 && a.splits <= 0 && !a.step && (int64_t)a.q_heads * a.nq >= PROMPT_FROM &&
-         (int64_t)(a.q_heads / a.heads) * a.nq >= PROMPT_ROWS;
+         (int64_t)(a.q_heads / a.heads) * a.nq >= PROMPT_ROWS && table_covers(a);
 }
 
 static PromptPlan make_prompt_plan(const dkv_attn_args& a) {

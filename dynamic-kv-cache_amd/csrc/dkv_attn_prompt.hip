@@ -133,19 +133,24 @@ prompt_tiles_kernel(dkv_attn_args a, uint8_t* __restrict__ images) {
   float2 ka = make_float2(0.f, 0.f), va = ka;
   if (r < hist) {
     const uint64_t before = ((uint64_t)starts[1] << 32 | starts[0]) & ((2ull << r) - 1);
-    const dkv_tile d = desc[first_tile + __builtin_popcountll(before)];
+    const int at = first_tile + __builtin_popcountll(before);  // (-1: no tile starts at or before the unit)
+    const dkv_tile d = desc[max(at, 0)];
     const int row = tok0 + r - d.token_start;
-    bits = d.bits;
-    const int64_t sb = subblock_bytes(d.rows, bits);
-    const uint8_t* ks = static_cast<const uint8_t*>(a.arena) + d.offset + ((int64_t)a.layer * 2 * a.heads + h) * sb;
-    const uint8_t* vs = ks + a.heads * sb;
-    const int rb = (int)row_bytes(bits);
-    if (bits != 16) {
-      ka = reinterpret_cast<const float2*>(ks + d.rows * rb)[row];
-      va = reinterpret_cast<const float2*>(vs + d.rows * rb)[row];
+    // The host saw a table that covers the history. A replay of a captured launch reads the device table of
+    // that time: a key it does not hold stays zero and is not read from past its tile.
+    if (at >= 0 && row >= 0 && row < (int)d.rows) {
+      bits = d.bits;
+      const int64_t sb = subblock_bytes(d.rows, bits);
+      const uint8_t* ks = static_cast<const uint8_t*>(a.arena) + d.offset + ((int64_t)a.layer * 2 * a.heads + h) * sb;
+      const uint8_t* vs = ks + a.heads * sb;
+      const int rb = (int)row_bytes(bits);
+      if (bits != 16) {
+        ka = reinterpret_cast<const float2*>(ks + d.rows * rb)[row];
+        va = reinterpret_cast<const float2*>(vs + d.rows * rb)[row];
+      }
+      kp = ks + row * rb + c * (rb >> 2);
+      vp = vs + row * rb + c * (rb >> 2);
     }
-    kp = ks + row * rb + c * (rb >> 2);
-    vp = vs + row * rb + c * (rb >> 2);
   } else if (tok0 + r < a.past + a.nq) {
     const int64_t j = tok0 + r - a.past;
     bits = 16;

@@ -109,12 +109,15 @@ typedef struct dkv_attn_args {
                             table. For a launch without `step` and n_tiles <= DKV_ARG_TILES the
                             frame-chunk kernel then takes the descriptors from its argument block
                             (read beside the arguments) instead of waiting on the device table
-                            before its first history loads; otherwise it is ignored. A copy whose
+                            before its first history loads. The long-chunk kernels (dkv_attend) run
+                            only where the copy shows a tile for every token below past, and read the
+                            device table. Otherwise it is ignored. A copy for the argument block whose
                             tiles are not well formed or do not cover [0, past) in token order is
                             refused (DKV_EINVAL). The descriptors are copied into the launch when
                             dkv_attend is called, so a launch captured in a HIP graph keeps the
                             ones it was captured with: its replays read the tiles as they were then
-                            (offsets, widths, rows), not the device table. Capture launches that
+                            (offsets, widths, rows), not the device table (long chunks do read that;
+                            a token it no longer holds counts as zeros). Capture launches that
                             must follow a table that changes (a cache reset, appends at other
                             widths) with `step`, or with tiles_host = NULL. */
 } dkv_attn_args;
@@ -208,8 +211,9 @@ int64_t dkv_attend_workspace_bytes(const dkv_attn_args* args);
  * packed_attention launch (src/gpu_cache.py:96-104, src/gpu_kernels.py:71-105).
  * Frames, candidate batches and decode steps run a split-history MFMA kernel
  * (path 0/2); long chunks (path 0, 4500 query rows or more over all Q heads, no
- * step pair and no explicit split count) unpack the keys once and run a causal
- * MFMA kernel over ranges of them (three launches);
+ * step pair, no explicit split count, and no history or a tiles_host that covers
+ * it) unpack the keys once and run a causal MFMA kernel over ranges of them (three
+ * launches);
  * path 3 runs short chunks (at most 16 query rows per KV head, e.g. decode
  * steps) on a kernel with two waves per 64-key tile. A merge kernel combines
  * the history splits of either in a second launch.

@@ -234,6 +234,33 @@ def test_attend_workspace_matches_the_partial_format():
         assert lib.dkv_attend_workspace_bytes(ctypes.byref(auto)) == (auto.heads * units * 3 * row if precision == 0 else big)
 
 
+@pytest.mark.parametrize('precision', [0, 1])
+def test_long_chunks_need_a_table_that_covers_their_history(precision):
+    """The long-chunk kernels look each history token up in the tile table; a call whose table cannot or
+    does not hold every token below past runs the plan of path 2, which walks the tiles there are."""
+    lib = _lib.load()
+
+    def need(tiles=None, **kw):
+        a = attn(**dict(dict(past=9600, n_tiles=150, arena=4096, tiles=4096, nq=2048, precision=precision), **kw))
+        if tiles is not None:
+            a.tiles_host = ctypes.addressof(tiles)
+        return lib.dkv_attend_workspace_bytes(ctypes.byref(a))
+
+    good = host_tiles([64] * 150)
+    long = need(good)
+    assert long > 5 * (9600 + 2048) * 256 and long != need(good, path=2)
+    assert need(good, past=9601) == need(good, past=9601, path=2)
+    assert need(good, past=9600, n_tiles=0) == need(good, n_tiles=0, path=2)
+    assert need(None) == need(None, path=2)  # no host copy to check
+    assert need(None, past=0, n_tiles=0) != need(None, past=0, n_tiles=0, path=2)  # no history to look up
+    for i, change in ((77, dict(rows=63)), (149, dict(rows=0)), (3, dict(token_start=191)), (20, dict(bits=5)),
+                      (0, dict(token_start=1)), (5, dict(rows=65)), (6, dict(offset=-16))):
+        bad = host_tiles([64] * 150)
+        for name, value in change.items():
+            setattr(bad[i], name, value)
+        assert need(bad) == need(bad, path=2), change
+
+
 def test_pack_validate_checks_every_job_of_a_host_table():
     lib = _lib.load()
     good = [job(seg_offset=0), job(seg_offset=4096, layer=1)]

@@ -278,6 +278,37 @@ def test_long_chunk_replays_equal_calls_as_replayed(cuda, past, nq, precision):
     c.end_graph_steps()
 
 
+def test_long_chunk_replay_over_a_shorter_table(cuda):
+    """A captured long chunk whose cache was reset and refilled with shorter tiles reads the device table of
+    that time: the ten tiles it was captured for now hold 100 of its 640 history tokens, and the rest count
+    as zeros, in every replay. Within the bounds of test_long_chunks_match_dense_attention."""
+    announce('routes: long chunk replay over a shorter table')
+    nq, past = 420, 640
+    case = frame_chunk_case(past, seed=8, nq=nq)
+    c, _ = filled(case, cuda, 5, precision='fp32')
+    q, k, v = (case[x][None].to(cuda) for x in ('q', 'k_new', 'v_new'))
+    c.attend(q, k, v, 0, past, out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = c.attend(q, k, v, 0, past, out_dtype=torch.float32)
+    hist_k, hist_v = case['k_hist'][None].to(cuda), case['v_hist'][None].to(cuda)
+    for bits in (4, 8, 16):
+        c.reset()
+        c.append_batch(hist_k, hist_v, [bits] * 64, [10] * 64)
+        graph.replay()
+        full_k, full_v = (x.clone() for x in c.materialize(0, torch.float32))
+        full_k[:, :, 100:], full_v[:, :, 100:] = 0, 0
+
+        class Held:
+            @staticmethod
+            def materialize(layer, dtype):
+                return full_k, full_v
+
+        ref, _ = _dense(Held, case, past, torch.zeros(nq, dtype=torch.long), torch.float32)
+        assert (out[0].double() - ref).abs().max() <= 1e-3, bits
+
+
 def test_long_chunk_without_scratch_for_its_keys(cuda):
     """dkv_attend_noalloc: the same call as dkv_attend where the unpacked keys and partials fit its
     scratch buffer; where they do not, the frame-chunk kernel's output instead of a refusal."""
