@@ -389,8 +389,11 @@ prompt_kernel(dkv_attn_args a, int units, int unit_len, int max_splits, int grou
       // The running maximum moves when some lane's scores pass it; only then do the four lanes of a
       // column exchange theirs. Precision 0 keeps the exact maximum, so that the largest p is 1 and
       // rounds to bf16 without error (moved only past 2^8, 2048 tokens past 8128 took 99.4 us instead
-      // of 101.8, but outputs were 7% further from exact ones); precision 1 moves it past 2^8.
-      if (__builtin_amdgcn_ballot_w64(t5 * xs > m_run[nb] + (PREC ? 8.f : 0.f))) {
+      // of 101.8, but outputs were 7% further from exact ones); precision 1 moves it past 2^6. (The
+      // frame-chunk kernel's two key groups each have a maximum and move it past 2^8. With 2^8 here 2048
+      // tokens past 1000 took 65.3 us instead of 65.7, but at 4.280e-6 from float64 where that kernel is
+      // at 4.218e-6; with 2^6 4.190e-6, and below that kernel at every size measured.)
+      if (__builtin_amdgcn_ballot_w64(t5 * xs > m_run[nb] + (PREC ? 6.f : 0.f))) {
         const float mnew = max_nn(m_run[nb], col_max(t5) * xs);
         const float alpha = mnew == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run[nb] - mnew);
         m_run[nb] = mnew;
