@@ -514,12 +514,17 @@ static Plan make_plan(const dkv_attn_args& a) {
 // split counts and paths keep the frame-chunk kernel) with PROMPT_FROM query rows over all Q heads and
 // a full workgroup of them per KV head. Their third launch and their unpacked keys cost about 8 us,
 // which the frame-chunk kernel's idle CUs, masked units and repeated dequantization pass from there
-// on; frame-chunk -> long-chunk kernels, us per call, bf16 (q_heads x nq rows):
-//   15 / 5 heads  3840 rows (256 past 1024) 16.4 -> 17.1   4800 (320 past 1024) 18.8 -> 17.3
-//   32 / 8 heads  3200 rows (100 past  500) 13.8 -> 15.2   6400 (200 past 1000) 22.0 -> 18.4
-//   16 / 8 heads  4096 rows (256 past 1024) 16.5 -> 17.3   8192 (512 past 1024) 24.0 -> 18.4
-//    9 / 3 heads  2880 rows (320 past 1024) 15.1 -> 16.2   4608 (512 past 1024) 18.1 -> 16.8
-static constexpr int64_t PROMPT_FROM = 4500;
+// on at every history; frame-chunk -> long-chunk kernels, us per call, past 0 / 1000 / 4000 / 20000:
+//   bf16  8 / 32 heads  4512 rows  14.9 -> 16.0   17.0 -> 18.5   25.4 -> 27.3   70.0 -> 60.9
+//                       6016 rows  15.7 -> 16.0   19.7 -> 19.2   29.4 -> 27.5   84.6 -> 62.3
+//         5 / 15 heads  4500 rows  15.3 -> 15.9   18.9 -> 18.2   25.8 -> 23.8   70.3 -> 54.6
+//                       6000 rows  16.1 -> 16.5   21.3 -> 18.8   31.2 -> 25.7   94.2 -> 60.6
+//         1 / 3 heads   6000 rows  21.4 -> 18.1   25.4 -> 20.6   34.9 -> 26.1   89.8 -> 56.8
+//   fp32  8 / 32 heads  4512 rows  18.1 -> 16.6   22.5 -> 23.0   32.5 -> 35.0   93.0 -> 106.8
+//                       6016 rows  19.0 -> 16.9   24.9 -> 23.7   36.8 -> 36.0  112.8 -> 111.0
+// (from 6000 rows on the worst of 7 head counts x 8 histories x 2 precisions: 66.2 -> 68.7, fp32, 8 / 32
+// heads, 7008 rows past 8128, whose ranges come out uneven).
+static constexpr int64_t PROMPT_FROM = 6000;
 // These kernels look every history token up in the tile table, where the frame-chunk kernel walks the
 // tiles there are and clamps each to its rows: they run only where the host copy of the table shows a tile
 // for each token below past (well under 1 ns per tile and call).

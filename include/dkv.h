@@ -210,7 +210,7 @@ int64_t dkv_attend_workspace_bytes(const dkv_attn_args* args);
 /* Fused packed-history causal GQA attention. Replaces GPUCache.attend's
  * packed_attention launch (src/gpu_cache.py:96-104, src/gpu_kernels.py:71-105).
  * Frames, candidate batches and decode steps run a split-history MFMA kernel
- * (path 0/2); long chunks (path 0, 4500 query rows or more over all Q heads, no
+ * (path 0/2); long chunks (path 0, 6000 query rows or more over all Q heads, no
  * step pair, no explicit split count, and no history or a tiles_host that covers
  * it) unpack the keys once and run a causal MFMA kernel over ranges of them (three
  * launches);

@@ -261,6 +261,27 @@ def test_long_chunks_need_a_table_that_covers_their_history(precision):
         assert need(bad) == need(bad, path=2), change
 
 
+@pytest.mark.parametrize('heads,q_heads,nq,long', [
+    (8, 32, 187, False), (8, 32, 188, True), (5, 15, 399, False), (5, 15, 400, True), (1, 3, 1999, False),
+    (1, 3, 2000, True), (60, 60, 255, False), (60, 60, 256, True),
+])
+@pytest.mark.parametrize('precision', [0, 1])
+def test_long_chunk_route_starts_where_it_is_faster(heads, q_heads, nq, long, precision):
+    """From 6000 query rows over all Q heads, and 256 per KV head, at any history; below, the plan of path 2
+    (at 4500 rows and short histories the long-chunk kernels were up to 9% slower)."""
+    lib = _lib.load()
+    for past in (0, 640, 20032):
+        arr = host_tiles([64] * (past // 64))
+        need = {}
+        for path in (0, 2):
+            a = attn(past=past, n_tiles=past // 64, arena=4096, tiles=4096, heads=heads, q_heads=q_heads, nq=nq,
+                     precision=precision, path=path)
+            if past:
+                a.tiles_host = ctypes.addressof(arr)
+            need[path] = lib.dkv_attend_workspace_bytes(ctypes.byref(a))
+        assert (need[0] != need[2]) == long
+
+
 def test_pack_validate_checks_every_job_of_a_host_table():
     lib = _lib.load()
     good = [job(seg_offset=0), job(seg_offset=4096, layer=1)]

@@ -122,14 +122,14 @@ def _dense(c, case, past, starts, dtype):
 
 
 @pytest.mark.parametrize('heads,group,nq,past,tiles', [
-    (5, 3, 300, 0, 'none'),         # no history; the first row sees one key
-    (5, 3, 301, 1, 'frames'),       # one key of history, an odd chunk
+    (5, 3, 400, 0, 'none'),         # no history; the first row sees one key
+    (5, 3, 401, 1, 'frames'),       # one key of history, an odd chunk
     (5, 3, 608, 999, 'frames'),     # past not a multiple of 64
     (8, 4, 256, 4096, 'frames'),    # the history ends on a unit
-    (8, 2, 282, 700, 'ones'),       # one-token tiles (decode steps), 700 of them: past the table window
-    (1, 1, 4500, 77, 'frames'),     # one head; the last group of rows is partly empty
-    (2, 8, 289, 5000, 'mixed'),     # tiles of 1 to 64 rows
-    (3, 3, 500, 64, 'frames'),
+    (8, 2, 378, 700, 'ones'),       # one-token tiles (decode steps), 700 of them: past the table window
+    (1, 1, 6010, 77, 'frames'),     # one head; the last group of rows is partly empty
+    (2, 8, 379, 5000, 'mixed'),     # tiles of 1 to 64 rows
+    (3, 3, 669, 64, 'frames'),
 ])
 @pytest.mark.parametrize('precision', ['bf16', 'fp32'])
 def test_long_chunks_match_dense_attention(cuda, heads, group, nq, past, tiles, precision):
@@ -139,7 +139,7 @@ def test_long_chunks_match_dense_attention(cuda, heads, group, nq, past, tiles, 
     exponentials take the rest of 2^-10); fp32: within 1e-3, as every fp32 path. The frame-chunk kernel
     (path='mfma') must agree with the same bounds, and two calls bit for bit."""
     announce(f'routes: long chunk heads={heads} group={group} nq={nq} past={past} tiles={tiles} {precision}')
-    assert heads * group * nq >= 4500 and group * nq >= 256
+    assert heads * group * nq >= 6000 and group * nq >= 256
     case = frame_chunk_case(past, seed=nq + past, heads=heads, q_heads=heads * group, nq=nq)
     c = GPUCache(None, layers=2, heads=heads, max_tokens=past + nq + 64, precision=precision)
     g = torch.Generator().manual_seed(past)
@@ -238,10 +238,10 @@ def test_long_chunk_partials_keep_large_values(cuda):
     """|V| near the top of bf16: the fp16 partial outputs are stored scaled; V and V * 2^20 give outputs
     that differ by exactly that factor, up to the one bit a scaled sum may lose (2^-15)."""
     announce('routes: long chunk, large values')
-    case = frame_chunk_case(2000, seed=9, nq=320)
+    case = frame_chunk_case(2000, seed=9, nq=420)
     outs = []
     for scale in (1.0, 2.0 ** 20):
-        c = GPUCache(None, layers=1, heads=5, max_tokens=2400)
+        c = GPUCache(None, layers=1, heads=5, max_tokens=2500)
         k, v = case['k_hist'][None].to(cuda), (case['v_hist'].float() * scale).to(torch.bfloat16)[None].to(cuda)
         c.append_batch(k, v, [16] * 32, [64] * 31 + [16])
         q, kn, vn = (case[x][None].to(cuda) for x in ('q', 'k_new', 'v_new'))
@@ -334,7 +334,7 @@ def test_long_chunk_without_scratch_for_its_keys(cuda):
     from dkv import _lib
     announce('routes: long chunk through dkv_attend_noalloc')
     lib = _lib.load()
-    for nq, past, fits in ((320, 1000, True), (2048, 30000, False)):
+    for nq, past, fits in ((420, 1000, True), (2048, 30000, False)):
         case = frame_chunk_case(past, seed=nq, nq=nq)
         c, past = filled(case, cuda, 5)
         q, k, v = (case[x][None].to(cuda) for x in ('q', 'k_new', 'v_new'))
