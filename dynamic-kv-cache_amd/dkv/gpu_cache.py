@@ -184,9 +184,10 @@ class GPUCache(_CacheBase):
         """_open_segment() of consecutive nonempty segments, all or none: the same bookkeeping, with the
         tile table filled in one go. Returns the index of the first new tile."""
         blocks = self.layers * 2 * self.heads
-        n, b = np.array(lengths, dtype=np.int64), np.array(bits, dtype=np.int64)
         block_of = {w: subblock_bytes(TILE, w) for w in BITS}
         full_block = np.array([block_of[w] for w in bits], dtype=np.int64)
+        n, b = np.array(lengths, dtype=np.int64), np.array(bits, dtype=np.int64)
+        lengths, bits = n.tolist(), b.tolist()  # plain ints for the bookkeeping
         row = full_block // TILE
         last = (n * row % (TILE * row) + 15) & ~15  # the partial tile's sub-block (0: none)
         need = (n // TILE * full_block + last) * blocks
@@ -476,7 +477,7 @@ class GPUCache(_CacheBase):
         if past + k.shape[2] > self.capacity:
             raise ValueError('GPU context limit exceeded')
         k, v = self._kv_view4(k), self._kv_view4(v)
-        if self.online and lengths and min(lengths) > 0:
+        if self.online and len(lengths) and min(lengths) > 0:
             tile0 = self._open_segments(past, lengths, bits, self.frame_id)
             batch = PackVolume(self, k, v, past, tile0)
             batch.run()

@@ -437,3 +437,18 @@ def test_volume_append_equals_appends(cuda, layers, heads, lengths, strided):
     a.arena[a.segments[1].offset:].zero_()
     batch.run()
     assert torch.equal(a.arena[:used], b.arena[:used])
+
+
+def test_volume_append_takes_arrays(cuda):
+    """lengths and bits as numpy arrays are what the same lists are, plain ints in the bookkeeping."""
+    import numpy as np
+    announce('routes: volume append, array arguments')
+    g = torch.Generator().manual_seed(5)
+    k, v = (torch.randn((2, 3, 200, 64), generator=g).to(torch.bfloat16).to(cuda) for _ in range(2))
+    a, b = (GPUCache(None, layers=2, heads=3, max_tokens=200) for _ in range(2))
+    for c in (a, b):
+        c.arena.zero_()
+    a.append_batch(k, v, [4, 8, 16], [64, 130, 6])
+    b.append_batch(k, v, np.array([4, 8, 16]), np.array([64, 130, 6]))
+    assert torch.equal(a.arena, b.arena) and a.plan == b.plan and a.seen == b.seen
+    assert all(type(x) is int for entry in b.plan for x in entry)

@@ -1,6 +1,7 @@
 """GPUCache._open_segments (the batch form append_batch uses) against _open_segment, one by one."""
 import random
 
+import numpy as np
 import pytest
 
 from dkv.gpu_cache import GPUCache
@@ -22,6 +23,8 @@ def test_batch_bookkeeping_equals_one_by_one(seed):
         for n, b in zip(lengths, bits):
             one._open_segment(at, n, b, frame)
             at += n
+        if seed % 2:  # arrays are what the same lists are
+            lengths, bits = np.array(lengths), np.array(bits)
         assert batch._open_segments(start, lengths, bits, frame) == tile0
         start = at
     for name in ('plan', 'tile_starts', 'host_counts', 'arena_used', 'arena_bytes'):
