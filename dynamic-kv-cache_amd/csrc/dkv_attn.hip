@@ -538,9 +538,17 @@ static bool table_covers(const dkv_attn_args& a) {
   }
   return next >= a.past;
 }
+// Most bytes of unpacked keys: a call past it runs the frame-chunk kernel in a few MB of partials. (4 GiB
+// holds two million tokens of 8 KV heads at precision 0; the packed tiles of one layer take a third to all
+// of what its unpacked keys do.)
+static constexpr int64_t PROMPT_MAX_IMAGES = (int64_t)4 << 30;
+static int64_t prompt_images(const dkv_attn_args& a) {
+  return (int64_t)a.heads * (((int64_t)a.past + a.nq + TILE - 1) / TILE) * prompt_image_bytes(a.precision);
+}
 static bool prompt_route(const dkv_attn_args& a) {
   return a.path == 0 && a.splits <= 0 && !a.step && (int64_t)a.q_heads * a.nq >= PROMPT_FROM &&
-         (int64_t)(a.q_heads / a.heads) * a.nq >= PROMPT_ROWS && table_covers(a);
+         (int64_t)(a.q_heads / a.heads) * a.nq >= PROMPT_ROWS &&
+         prompt_images(a) <= PROMPT_MAX_IMAGES && table_covers(a);
 }
 
 static PromptPlan make_prompt_plan(const dkv_attn_args& a) {

@@ -148,7 +148,7 @@ class GPUCache(_CacheBase):
         self.tiles_host = np.zeros(self.tiles.shape[0], dtype=TILE_DTYPE)
         self._tiles_host_ptr = self.tiles_host.ctypes.data  # fixed: the array is never replaced
         self._tiles_host_bytes = self.tiles_host.view(np.uint8)
-        self._workspace = None  # split partials of the last call that needed any
+        self._workspace = None  # bytes of workspace the last call that needed any took
         self._graph = None  # GraphSteps while launches read their step parameters from the device
         self._fused_args, self._fused_key = None, None  # the argument block _fused_attention() reuses
         for bits, n in planned:
@@ -542,9 +542,10 @@ class GPUCache(_CacheBase):
         # need no clearing. A block of its own for every call, from torch's allocator (stream-ordered
         # reuse): calls on several streams or threads never share one. Clearing it cost a launch of its
         # own, 2.4-4.6 us of GPU time beside the 8.6 us of a decode step's two kernels.
+        # The cache keeps no reference: the block (megabytes for a long chunk) goes back with the call.
         alloc = self.arena.new_empty if _lib.workspace_uncleared() else self.arena.new_zeros
-        self._workspace = ws = alloc(nbytes)
-        return ws
+        self._workspace = nbytes
+        return alloc(nbytes)
 
     def attend(self, q, k, v, layer, past, out_dtype=None, segments=None, path=0, splits=0, precision=None):
         """Causal attention of q over history [0, past) plus the native chunk (src/gpu_cache.py:96-104).

@@ -204,7 +204,8 @@ int dkv_reconstruct(const void* arena, const dkv_tile* tiles, int32_t n_tiles,
                     void* out, int32_t out_dtype, void* stream);
 
 /* Workspace bytes dkv_attend needs for these arguments: the split partials, and for a long chunk
- * (path 0) its keys unpacked, heads * (past + nq) * 256 bytes (512 at precision 1). */
+ * (path 0) its keys unpacked, heads * (past + nq) * 256 bytes (512 at precision 1), at most 4 GiB
+ * (calls beyond that run the frame-chunk kernel). */
 int64_t dkv_attend_workspace_bytes(const dkv_attn_args* args);
 
 /* Fused packed-history causal GQA attention. Replaces GPUCache.attend's

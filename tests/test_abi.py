@@ -282,6 +282,20 @@ def test_long_chunk_route_starts_where_it_is_faster(heads, q_heads, nq, long, pr
         assert (need[0] != need[2]) == long
 
 
+def test_long_chunk_workspace_is_bounded():
+    """The unpacked keys grow with the history; past 4 GiB the call runs the plan of path 2."""
+    lib = _lib.load()
+    for heads, past, precision in ((8, 64 * 33000, 0), (8, 64 * 16500, 1), (64, 64 * 4100, 0)):
+        arr = host_tiles([64] * (past // 64))
+        need = {}
+        for path in (0, 2):
+            a = attn(past=past, n_tiles=past // 64, arena=4096, tiles=4096, nq=512, precision=precision, path=path,
+                     heads=heads, q_heads=2 * heads)
+            a.tiles_host = ctypes.addressof(arr)
+            need[path] = lib.dkv_attend_workspace_bytes(ctypes.byref(a))
+        assert need[0] == need[2] < 2 ** 28
+
+
 def test_pack_validate_checks_every_job_of_a_host_table():
     lib = _lib.load()
     good = [job(seg_offset=0), job(seg_offset=4096, layer=1)]

@@ -452,3 +452,15 @@ def test_volume_append_takes_arrays(cuda):
     b.append_batch(k, v, np.array([4, 8, 16]), np.array([64, 130, 6]))
     assert torch.equal(a.arena, b.arena) and a.plan == b.plan and a.seen == b.seen
     assert all(type(x) is int for entry in b.plan for x in entry)
+
+
+def test_attend_returns_its_workspace(cuda):
+    """The workspace of a call (megabytes for a long chunk) goes back to the allocator with it; the cache
+    keeps none of it."""
+    announce('routes: workspace given back')
+    case = frame_chunk_case(1000, seed=4, nq=1000)
+    c, past = filled(case, cuda, 5)
+    q, k, v = (case[x][None].to(cuda) for x in ('q', 'k_new', 'v_new'))
+    held = torch.cuda.memory_allocated()
+    out = c.attend(q, k, v, 0, past)
+    assert torch.cuda.memory_allocated() - held <= out.numel() * 2 + 4096
