@@ -30,6 +30,7 @@ BITS = (4, 8, 16)
 # does (src/gpu_kernels.py:93-94,102). 'fp32': fp32-accurate (split bf16 pairs on the MFMA path).
 PRECISIONS = {'bf16': 0, 'fp32': 1}
 PATHS = {'auto': 0, 'vector': 1, 'mfma': 2, 'short': 3}
+WORKSPACE_KEPT = 128 << 20  # bytes of attention workspace a cache holds from one call to the next, at most
 _ONE_SEGMENT = (0,) * (_lib.DKV_MAX_CHUNK_SEGS + 1)  # dkv_attn_args.seg_bounds of an unsegmented chunk
 SMALL_ROWS = 32  # query rows per KV head up to which 'auto' runs the decode-step variant (MFMA_SMALL_ROWS there)
 SHORT_ROWS = 16  # query rows per KV head the short-chunk kernel takes (SHORT_ROWS of csrc/dkv_attn_common.h)
@@ -148,7 +149,7 @@ class GPUCache(_CacheBase):
         self.tiles_host = np.zeros(self.tiles.shape[0], dtype=TILE_DTYPE)
         self._tiles_host_ptr = self.tiles_host.ctypes.data  # fixed: the array is never replaced
         self._tiles_host_bytes = self.tiles_host.view(np.uint8)
-        self._workspace = None  # bytes of workspace the last call that needed any took
+        self._workspace = None  # the last call's workspace, up to WORKSPACE_KEPT bytes (_workspace_for)
         self._graph = None  # GraphSteps while launches read their step parameters from the device
         self._fused_args, self._fused_key = None, None  # the argument block _fused_attention() reuses
         for bits, n in planned:
@@ -542,10 +543,14 @@ class GPUCache(_CacheBase):
         # need no clearing. A block of its own for every call, from torch's allocator (stream-ordered
         # reuse): calls on several streams or threads never share one. Clearing it cost a launch of its
         # own, 2.4-4.6 us of GPU time beside the 8.6 us of a decode step's two kernels.
-        # The cache keeps no reference: the block (megabytes for a long chunk) goes back with the call.
+        # The cache holds a block until its next call has its own, so that two alternate: a call that wrote
+        # the bytes the call before it had just read took longer (2048 tokens past 1000 48.0 us instead of
+        # 45.0, 4096 tokens 69.2 instead of 66.1). Blocks over WORKSPACE_KEPT, where that is 2%, go back
+        # with the call.
         alloc = self.arena.new_empty if _lib.workspace_uncleared() else self.arena.new_zeros
-        self._workspace = nbytes
-        return alloc(nbytes)
+        ws = alloc(nbytes)
+        self._workspace = ws if nbytes <= WORKSPACE_KEPT else None
+        return ws
 
     def attend(self, q, k, v, layer, past, out_dtype=None, segments=None, path=0, splits=0, precision=None):
         """Causal attention of q over history [0, past) plus the native chunk (src/gpu_cache.py:96-104).

@@ -454,13 +454,18 @@ def test_volume_append_takes_arrays(cuda):
     assert all(type(x) is int for entry in b.plan for x in entry)
 
 
-def test_attend_returns_its_workspace(cuda):
-    """The workspace of a call (megabytes for a long chunk) goes back to the allocator with it; the cache
-    keeps none of it."""
+def test_attend_holds_little_workspace(cuda):
+    """The workspace of a call goes back to the allocator with it when it is large (a long chunk's unpacked
+    keys); of a smaller one the cache holds the last, at most WORKSPACE_KEPT bytes."""
+    from dkv.gpu_cache import WORKSPACE_KEPT
     announce('routes: workspace given back')
-    case = frame_chunk_case(1000, seed=4, nq=1000)
-    c, past = filled(case, cuda, 5)
-    q, k, v = (case[x][None].to(cuda) for x in ('q', 'k_new', 'v_new'))
-    held = torch.cuda.memory_allocated()
-    out = c.attend(q, k, v, 0, past)
-    assert torch.cuda.memory_allocated() - held <= out.numel() * 2 + 4096
+    for past, nq in ((52000, 1000), (1000, 1000)):
+        case = frame_chunk_case(past, seed=4, nq=nq)
+        c, past = filled(case, cuda, 5, precision='fp32')
+        q, k, v = (case[x][None].to(cuda) for x in ('q', 'k_new', 'v_new'))
+        assert (5 * (past + nq) * 512 > WORKSPACE_KEPT) == (past > 20000)
+        held = torch.cuda.memory_allocated()
+        for _ in range(3):
+            out = c.attend(q, k, v, 0, past)
+        kept = torch.cuda.memory_allocated() - held - out.numel() * 2
+        assert kept <= (4096 if past > 20000 else WORKSPACE_KEPT + 4096)
