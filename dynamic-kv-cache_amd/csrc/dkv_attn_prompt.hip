@@ -242,15 +242,6 @@ __device__ __forceinline__ float col_sum(float x) {
   return __uint_as_float(q[0]) + __uint_as_float(q[1]);
 }
 
-// One 1 KB piece per call: lane l's 16 bytes from `from` (per lane) to LDS byte `to` + 16 l. The
-// instruction is written out because the compiler, knowing that a global_load_lds builtin writes
-// LDS, makes ordinary LDS reads wait for every one in flight. It has no register output; the waits
-// below count it. (M0, the LDS base, is set and used within the statement; an LDS load wants one
-// instruction between the two, and the compiler adds none inside a statement.)
-__device__ __forceinline__ void load_piece(const uint8_t* from, uint32_t to) {
-  asm volatile("s_mov_b32 m0, %1\n s_nop 0\n global_load_lds_dwordx4 %0, off" ::"v"(from), "s"(to) : "memory");
-}
-
 // HALF: the partials of groups with several ranges, see PromptPlan::half.
 template <int PREC, bool HALF>
 __global__ void __launch_bounds__(64 * PROMPT_WAVES, 4)

@@ -75,6 +75,18 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
 // x rounded to the nearest bf16 value, as fp32.
 __device__ __forceinline__ float round_bf16(float x) { return bf16_lo(pack_bf16(x, 0.f)); }
 
+// A 1 KB piece straight to LDS: lane l's 16 bytes from `from` (per lane) go to LDS byte `to` + 16 l. The
+// instruction is written out because the compiler, knowing that a global_load_lds builtin writes LDS, makes
+// ordinary LDS reads wait for every one in flight. It has no register output; the callers' waits count it.
+// M0, the LDS base, is put back: it cannot be named as clobbered (the compiler keeps it to itself), and what
+// the compiler holds there must outlive the statement. An LDS load wants one instruction between M0's write
+// and itself, which the compiler does not add inside a statement.
+__device__ __forceinline__ void load_piece(const void* from, uint32_t to) {
+  uint32_t m0;
+  asm volatile("s_mov_b32 %0, m0\n s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %1, off\n s_mov_b32 m0, %0"
+               : "=&s"(m0) : "v"(from), "s"(to) : "memory");
+}
+
 // Thread-local message for DKV_EINVAL returns.
 void set_error(const char* fmt, ...);
 void clear_error();

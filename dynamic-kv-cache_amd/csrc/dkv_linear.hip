@@ -685,8 +685,7 @@ __global__ void __launch_bounds__(256, 3) linear_glu_kernel(const LinearArgs a) 
       for (int h = 0; h < 2; ++h) to[nb][h].u = *reinterpret_cast<const u32x4*>(wsrc[nb] + wsp * pl + wsh * h);
 #pragma unroll
     for (int q = 0; q < XW; ++q)
-      asm volatile("s_mov_b32 m0, %1\n s_nop 0\n global_load_lds_dwordx4 %0, off" ::"v"(xsrc[q] + (x_tiled ? 1024 : 64) * pl),
-                   "s"(lds0 + 1024 * (fill * XF + wave + 4 * q)) : "memory");
+      load_piece(xsrc[q] + (x_tiled ? 1024 : 64) * pl, lds0 + 1024 * (fill * XF + wave + 4 * q));
     fill = fill + 1 == GLU_RING ? 0 : fill + 1;
     if (++loaded < a.kp) pl = next(pl);
   };
