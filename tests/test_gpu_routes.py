@@ -468,4 +468,5 @@ def test_attend_holds_little_workspace(cuda):
         for _ in range(3):
             out = c.attend(q, k, v, 0, past)
         kept = torch.cuda.memory_allocated() - held - out.numel() * 2
-        assert kept <= (4096 if past > 20000 else WORKSPACE_KEPT + 4096)
+        # (torch's allocator leaves up to 1 MiB of a block unsplit: of the output's, of the one held)
+        assert kept <= (0 if past > 20000 else WORKSPACE_KEPT + 2 ** 20) + 2 ** 20
