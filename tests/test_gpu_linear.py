@@ -170,6 +170,75 @@ def test_fused_layers_match_upstream_layers(cuda):
     assert diff <= 0.05, diff
 
 
+@pytest.mark.parametrize('n', [97, 131, 353, 701, 999])
+@pytest.mark.parametrize('tiled', [True, False])
+def test_fused_layer_of_many_rows(cuda, n, tiled):
+    """fused_decoder_layer of the 960-wide decoder at row counts where gate/up's norm (from 97 rows) and
+    Q/K/V's (from 353) are launches of their own, on tiled and row-major weights. Against the upstream layer
+    forward (library projections, one launch per op): a flipped bf16 rounding of one input moves an output
+    by 2^-8 of one term in 960, so 2-norms within 0.4% (5e-4 to 1e-3 seen). Against the same layer recorded
+    with graph steps, which runs other launches: the same bits of output and cache, in every replay."""
+    announce(f'linear: fused layer of {n} rows, tiled weights {tiled}')
+    from dkv.gpu_cache import GPUCache
+    from dkv.streaming import StreamingDecoder, build_decoder
+    dec = StreamingDecoder(build_decoder(layers=1, vocab=64, seed=n), precision='fp32')
+    layer = dec.text.layers[0]
+    p = gpu_ops._layer_plan(layer, n, 960)
+    assert (p.norm1_apart, p.norm2_apart) == (n >= 353, True)
+    g = torch.Generator().manual_seed(n)
+    hidden = [torch.randn((1, n, 960), generator=g).to(BF).to(cuda) for _ in range(2)]
+    lead = torch.randn((1, 5, 100, 64), generator=g).to(BF).to(cuda)
+
+    def cache():
+        c = GPUCache(None, layers=1, heads=5, max_tokens=100 + 2 * n, precision='fp32')
+        c.arena.zero_()
+        c.select(8)
+        c.append(lead, lead, 0)
+        c.select(16)
+        c.as_replayed = True
+        return c
+
+    def rope(at):
+        with torch.inference_mode():
+            return dec.text.rotary_emb(hidden[0], torch.arange(at, at + n, device=cuda)[None])
+
+    orig = gpu_ops._layer_tiles
+    if not tiled:
+        gpu_ops._layer_tiles = lambda layer, p: None
+    try:
+        with torch.inference_mode():
+            eager, upstream = cache(), cache()
+            got = [gpu_ops.fused_decoder_layer(layer, h, eager, rope(100 + i * n)) for i, h in enumerate(hidden)]
+            dec.ops_state['layers'] = False
+            want = [layer(h, past_key_values=upstream, position_embeddings=rope(100 + i * n), attention_mask=None)
+                    for i, h in enumerate(hidden)]
+            dec.ops_state['layers'] = True
+            for a, b in zip(got + list(eager.materialize(0)), want + list(upstream.materialize(0))):
+                assert a.shape == b.shape and (a.float() - b.float()).norm() <= 0.004 * b.float().norm()
+            c = cache()
+            steps = c.begin_graph_steps(n, q_heads=15)
+            c.graph_step()
+            h, (cos, sin) = hidden[0].clone(), rope(100)
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                out = gpu_ops.fused_decoder_layer(layer, h, c, (cos, sin))
+            steps.upload()
+            for i in range(2):
+                if i:
+                    c.graph_step()
+                    h.copy_(hidden[i])
+                    for dst, src in zip((cos, sin), rope(100 + i * n)):
+                        dst.copy_(src)
+                graph.replay()
+                assert torch.equal(out, got[i])
+            c.end_graph_steps()
+            assert torch.equal(c.arena, eager.arena) and c.plan == eager.plan
+    finally:
+        gpu_ops._layer_tiles = orig
+        dec.ops_state['layers'] = True
+
+
 def test_eager_fused_layers_follow_weight_changes(cuda):
     """The eager fused layers check a layer once per chunk length and keep its weight objects, reading
     their data pointers at every call: a weight whose storage moves (param.data replaced, as
