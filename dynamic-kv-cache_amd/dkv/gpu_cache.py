@@ -407,16 +407,15 @@ class GPUCache(_CacheBase):
         project = (x.data_ptr(), x.stride(0), weight.data_ptr(), weight_stride, n, x.shape[1], norm.data_ptr(), eps, layout)
         return q, k, v, self._graph.append_hidden(project, cos, sin, q_heads, layer, q, k, v)
 
-    def _fused_attention(self, n, q_heads, layer, qkv, qkv_stride, cos, sin, cs_stride, qkv_out, out, stream,
-                         project=None):
-        """append_projection() then attend() for the fused decoder layer's eager launches: the same
-        two launches with the same arguments (so the same bytes and outputs), without the per-call
-        checks of the general entry points, which cost more host time than the GPU spends on a
-        64-token chunk. Raw device addresses, which the caller guarantees to be what those checks
-        establish: qkv [n, (q_heads + 2 heads) * 64] and cos / sin [n, 64] bf16 rows (element
-        strides qkv_stride, cs_stride), qkv_out room for q | k | v as [heads, n, 64] blocks and out
-        for the bf16 output [1, n, q_heads, 64], all 16-byte aligned; no graph steps (eager
-        launches) and no chunk segments."""
+    def _fused_attention(self, n, q_heads, layer, project, cos, sin, cs_stride, qkv_out, out, stream):
+        """The joined Q/K/V projection, append_projection() and attend() for the fused decoder layer's
+        eager launches: the same bytes and outputs, without the per-call checks of the general entry
+        points, which cost more host time than the GPU spends on a 64-token chunk. `project` holds
+        dkv_linear_rope_pack's first arguments (x, its row stride, weight, its row stride, rows, k,
+        norm weight, eps, layout). Raw device addresses, which the caller guarantees to be what those
+        checks establish: cos / sin [n, 64] bf16 rows (element stride cs_stride), qkv_out room for
+        q | k | v as [heads, n, 64] blocks and out for the bf16 output [1, n, q_heads, 64], all 16-byte
+        aligned; no graph steps (eager launches) and no chunk segments."""
         H, d = self.heads, self.dim
         past, seg, write_tiles = self._claim(layer, n)
         kp = qkv_out + q_heads * n * d * 2
@@ -425,14 +424,9 @@ class GPUCache(_CacheBase):
         job = _lib.PackJob(kp, vp, head, d, head, d, seg.offset, seg.rows, seg.start, past - seg.start,
                            n, layer, seg.bits, seg.tile0, write_tiles)
         lib = _lib.load()
-        if project is not None:
-            _lib.check(lib.dkv_linear_rope_pack(*project, cos, sin, cs_stride, q_heads, qkv_out, kp, vp,
-                                                ctypes.byref(job), 0, self.arena.data_ptr(), self.arena_bytes,
-                                                self.tiles.data_ptr(), self.layers, H, stream), 'dkv_linear_rope_pack')
-        else:
-            _lib.check(lib.dkv_rope_pack(qkv, qkv_stride, cos, sin, cs_stride, n, q_heads, qkv_out, kp, vp,
-                                         ctypes.byref(job), 0, self.arena.data_ptr(), self.arena_bytes,
-                                         self.tiles.data_ptr(), self.layers, H, stream), 'dkv_rope_pack')
+        _lib.check(lib.dkv_linear_rope_pack(*project, cos, sin, cs_stride, q_heads, qkv_out, kp, vp,
+                                            ctypes.byref(job), 0, self.arena.data_ptr(), self.arena_bytes,
+                                            self.tiles.data_ptr(), self.layers, H, stream), 'dkv_linear_rope_pack')
         self.seen[layer] = past + n
         a = self._fused_args
         if a is None or self._fused_key != (n, q_heads):

@@ -217,7 +217,7 @@ class _LayerPlan:
     epsilons and the head counts."""
     __slots__ = ('qkv_w', 'o_w', 'gu_w', 'd_w', 'ln1_w', 'ln2_w', 'qkv_args', 'o_args', 'gu_args', 'd_args',
                  'eps1', 'eps2', 'q_heads', 'kv_heads', 'eager_ok', 'layer_idx', 'width', 'inter', 'norm1_apart',
-                 'norm2_apart', 'rope_in_qkv')
+                 'norm2_apart')
 
     def holds(self, layer):
         # the modules' own dicts: nn.Module attribute lookups cost more than the rest of this check
@@ -294,25 +294,24 @@ def _layer_plan(layer, n, width):
     p.d_args = (d_w, d_w.stride(0), d_w.shape[0], d_w.shape[1])
     sizes, hd = attn._qkv_sizes, attn.head_dim
     p.q_heads, p.kv_heads = sizes[0] // hd, sizes[1] // hd
-    # the eager launches split q | k | v as dkv_rope_pack does: 64-wide heads, K and V alike
+    # Q/K/V goes on to RoPE and the pack in its own launch (dkv_linear_rope_pack, faster at every size,
+    # see the kernels), which splits q | k | v as dkv_rope_pack does: 64-wide heads, K and V alike
     p.eager_ok = hd == 64 and sizes[1] == sizes[2] and p.qkv_w.shape[0] == sum(sizes) and sizes[0] % hd == 0
     p.layer_idx, p.width, p.inter = attn.layer_idx, width, p.gu_w.shape[0] // 2
     # many rows: the norms as launches of their own, before Q/K/V and gate/up
     p.norm1_apart = _prenorm(n, p.qkv_w.shape[0], width, LINEAR_PLAIN)
     p.norm2_apart = _prenorm(n, p.gu_w.shape[0], width, LINEAR_SILU_MUL)
-    # Q/K/V goes on to RoPE and the pack in its own launch (faster at every size, see the kernels)
-    p.rope_in_qkv = p.eager_ok and n > 0
     plans[(n, width)] = p
     return p
 
 
 def _fused_layer_eager(p, tiles, h, n, cache, cos, sin):
-    """The fused layer's eager launches for a checked plan: the launches and arguments linear() and
-    attend_projection() would make, without their per-call checks (which cost more host time than
-    the GPU spends on a 64-token chunk). The intermediates (the joined projection, q | k | v, the
-    attention output, the post-attention residual, SiLU*up) share one allocation; the kernels read
-    and write it in stream order, and the allocator hands it out again only to later work on the
-    same stream."""
+    """The fused layer's eager launches for a checked plan: what linear() and attend_projection()
+    would compute, bit for bit, with Q/K/V, RoPE and the pack in one launch and without their per-call
+    checks (which cost more host time than the GPU spends on a 64-token chunk). The intermediates
+    (q | k | v, the attention output, the post-attention residual, SiLU*up, the normalized rows where
+    a norm is a launch of its own) share one allocation; the kernels read and write it in stream
+    order, and the allocator hands it out again only to later work on the same stream."""
     lib = _lib.load()
     stream = _lib.stream_handle(h.device)
     width, inter = p.width, p.inter
@@ -331,32 +330,25 @@ def _fused_layer_eager(p, tiles, h, n, cache, cos, sin):
             ol |= LINEAR_OUT_TILED
             gl |= LINEAR_X_TILED
             dl |= LINEAR_RES_TILED
-    # element offsets of [qkv | q,k,v | attention out | h2 | act], each n rows (multiples of 64
-    # columns; h2 and act in rows rounded up to 16 when tiled)
-    o_qkvo = n * qrows
-    o_att = o_qkvo + n * qrows
+    # element offsets of [q,k,v | attention out | h2 | act | normalized rows], each n rows (multiples
+    # of 64 columns; h2, act and the normalized rows in rows rounded up to 16, as their tiles are)
+    o_att = n * qrows
     o_h2 = o_att + n * ok
     n16 = (n + 15) // 16 * 16
     o_act = o_h2 + n16 * orows
-    o_norm = o_act + n16 * inter  # the normalized rows, tiled, where a norm is a launch of its own
+    o_norm = o_act + n16 * inter
     apart = p.norm1_apart or p.norm2_apart
     scratch = torch.empty(o_norm + (n16 * width if apart else 0), dtype=torch.bfloat16, device=h.device)
     out = torch.empty((1, n, drows), dtype=torch.bfloat16, device=h.device)
     base = scratch.data_ptr()
-    xp, qkv, att, h2, act = h.data_ptr(), base, base + 2 * o_att, base + 2 * o_h2, base + 2 * o_act
+    xp, att, h2, act = h.data_ptr(), base + 2 * o_att, base + 2 * o_h2, base + 2 * o_act
     xn = base + 2 * o_norm
     qx, norm1 = xp, p.ln1_w.data_ptr()
     if p.norm1_apart:
         _lib.check(lib.dkv_rms_norm_tiled(xp, width, norm1, xn, n, width, p.eps1, 0, stream), 'dkv_rms_norm_tiled')
         qx, norm1, ql = xn, None, ql | LINEAR_X_TILED
-    project = None
-    if p.rope_in_qkv:  # RoPE and the pack in the projection's launch
-        project = (qx, width, qw.data_ptr(), qld, n, qk, norm1, p.eps1, ql)
-    else:
-        _lib.check(lib.dkv_linear_tiled(qx, width, qw.data_ptr(), qld, n, qrows, qk, norm1, p.eps1,
-                                        LINEAR_PLAIN, None, 0, qkv, qrows, ql, stream), 'dkv_linear')
-    cache._fused_attention(n, p.q_heads, p.layer_idx, qkv, qrows, cos.data_ptr(), sin.data_ptr(), cos.stride(0),
-                           base + 2 * o_qkvo, att, stream, project)
+    cache._fused_attention(n, p.q_heads, p.layer_idx, (qx, width, qw.data_ptr(), qld, n, qk, norm1, p.eps1, ql),
+                           cos.data_ptr(), sin.data_ptr(), cos.stride(0), base, att, stream)
     _lib.check(lib.dkv_linear_tiled(att, ok, ow.data_ptr(), old, n, orows, ok, None, 1e-6, LINEAR_RESIDUAL, xp,
                                     width, h2, orows, ol, stream), 'dkv_linear')
     gx, norm2 = h2, p.ln2_w.data_ptr()
@@ -372,10 +364,12 @@ def _fused_layer_eager(p, tiles, h, n, cache, cos, sin):
 
 
 def fused_decoder_layer(layer, hidden_states, cache, position_embeddings):
-    """One LlamaDecoderLayer forward on a packed GPUCache as four or five launches plus the attention's
-    two; None when the layer, the inputs or the cache are outside what they cover. What depends
-    only on the layer and the chunk length is checked once (_layer_plan); eager launches on
-    contiguous inputs then take _fused_layer_eager, and graph captures the general path below."""
+    """One LlamaDecoderLayer forward on a packed GPUCache; None when the layer, the inputs or the cache
+    are outside what the kernels cover. Launches beside the attention's (one to three): four, up to six
+    where the norms run apart (many rows), one more in graph steps of so many rows that the norm before
+    Q/K/V is apart, which rotate and pack in a launch of their own. What depends only on the layer and
+    the chunk length is checked once (_layer_plan); eager launches on contiguous inputs then take
+    _fused_layer_eager, and graph captures the general path below."""
     from .gpu_cache import GPUCache, attend_projection
     attn, mlp = layer._modules['self_attn'], layer._modules['mlp']
     h = hidden_states
@@ -399,7 +393,7 @@ def fused_decoder_layer(layer, hidden_states, cache, position_embeddings):
     x = h.reshape(n, width)
     qt, ot, gt, dt = tiles if tiles is not None else (None,) * 4
     packed = None
-    if p.rope_in_qkv and not p.norm1_apart and p.kv_heads == cache.heads and cache._graph is not None:
+    if p.eager_ok and not p.norm1_apart and p.kv_heads == cache.heads and cache._graph is not None:
         cos, sin = position_embeddings
         if (x.stride(-1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and cos.shape == (1, n, 64)
                 and sin.shape == cos.shape and all(t.is_cuda and t.dtype == torch.bfloat16 and t.stride(-1) == 1
