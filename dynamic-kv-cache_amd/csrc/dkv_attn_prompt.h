@@ -6,11 +6,14 @@ namespace dkv {
 
 constexpr int PROMPT_WAVES = 8;                 // per workgroup, each 32 tokens of one Q head
 constexpr int PROMPT_ROWS = 32 * PROMPT_WAVES;  // query rows of one KV head per workgroup
-// Ranges come to one workgroup per CU, or to two (which overlap each other's waits, but twice the
-// partials to merge) when there are at least this many units of 256 rows x 64 keys per CU. One against
-// two per CU, us per call (15 Q / 5 KV heads): 4 units per CU (1000 tokens past 640) 23.8 / 25.5, 15
-// (512 past 8128) 36.5 / 39.8, 16 (2048 past 1000) 40.2 / 39.4, 32 (1000 past 8128) 58.6 / 57.1, 67
-// (2048 past 8128) 106.4 / 100.1.
+// Ranges come to one workgroup per CU, or to two (twice the partials to merge) when there are at least
+// this many units of 256 rows x 64 keys per CU. One against two per CU, us per call (15 Q / 5 KV heads,
+// bf16): 4 units per CU (1000 tokens past 640) 23.8 / 25.5, 15 (512 past 8128) 36.5 / 39.8, 16 (2048 past
+// 1000) 40.2 / 39.4, 32 (1000 past 8128) 58.6 / 57.1, 67 (2048 past 8128) 106.4 / 100.1. At precision 0 two
+// workgroups share a CU (48 KB of LDS each) and overlap each other's waits. At precision 1 (96 KB) only one
+// fits and the second half runs after the first, which still evens out ranges of unequal length: 2048 past
+// 1000 64.8 / 65.1, 900 past 500 (32 / 8 heads) 42.9 / 42.6, 8192 tokens 287 / 287, 2048 past 8128
+// 193.8 / 189.5.
 constexpr int PROMPT_TWO_FROM = 16;
 constexpr int PROMPT_MIN_LEN = 2;  // units per range, at least (512 tokens past 1024: 4 units 20.5 us, 2 units 19.7)
 

@@ -595,8 +595,8 @@ PromptPlan prompt_plan(const dkv_attn_args& a, int cus, bool half) {
   p.units = (int)(((int64_t)a.past + a.nq + TILE - 1) / TILE);
   int64_t total = 0;
   for (int i = 0; i < p.groups; ++i) total += prompt_group_units(i, G, a.nq, a.past);
-  // One round of workgroups, all resident at once: the shortest ranges of which there are no more than
-  // slots (a few more would take a second round as long as the first). Chunks of more groups than
+  // One round of workgroups, all resident at once (two rounds at precision 1 from PROMPT_TWO_FROM on): the
+  // shortest ranges of which there are no more than slots (a few more would take another round as long). Chunks of more groups than
   // that take as many rounds as it needs for several ranges per slot.
   int64_t slots = (int64_t)(total * a.heads >= (int64_t)PROMPT_TWO_FROM * cus ? 2 : 1) * cus;
   if ((int64_t)p.groups * a.heads * 4 > slots * 3) slots *= ((int64_t)p.groups * a.heads * 2 + slots - 1) / slots;
