@@ -90,7 +90,8 @@ def time_launches(fn, steps, warmup):
     return start.elapsed_time(end) / steps  # ms per launch
 
 
-PACK_SOURCES = ('dynamic-kv-cache_amd/csrc/dkv_pack.hip', 'dynamic-kv-cache_amd/csrc/dkv_common.h')
+PACK_SOURCES = tuple(f'dynamic-kv-cache_amd/csrc/{f}'
+                     for f in ('dkv_pack.hip', 'dkv_common.h', 'dkv_rope_pack.h', 'dkv_attn_common.h'))
 
 
 def pack_source_hash():
