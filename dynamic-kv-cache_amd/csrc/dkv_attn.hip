@@ -511,20 +511,30 @@ static Plan make_plan(const dkv_attn_args& a) {
 }
 
 // Calls that take the long-chunk kernels (dkv_attn_prompt.hip): default plans (graph replays, explicit
-// split counts and paths keep the frame-chunk kernel) with PROMPT_FROM query rows over all Q heads and
-// a full workgroup of them per KV head. Their third launch and their unpacked keys cost about 8 us,
-// which the frame-chunk kernel's idle CUs, masked units and repeated dequantization pass from there
-// on at every history; frame-chunk -> long-chunk kernels, us per call, past 0 / 1000 / 4000 / 20000:
+// split counts and paths keep the frame-chunk kernel) of enough query rows over all Q heads, with a full
+// workgroup of them per KV head. Their third launch and their unpacked keys cost about 8 us, which the
+// frame-chunk kernel's idle CUs, masked units and repeated dequantization pass from 5500 rows on; from 5000
+// where a KV head has the rows of nearly four of its 256-row groups (with fewer, more of the last group is
+// empty); from 4500 then with a history to unpack once. Frame-chunk -> long-chunk kernels, us per call, past
+// 0 / 1000 / 4000 / 20000:
 //   bf16  8 / 32 heads  4512 rows  14.9 -> 16.0   17.0 -> 18.5   25.4 -> 27.3   70.0 -> 60.9
 //                       6016 rows  15.7 -> 16.0   19.7 -> 19.2   29.4 -> 27.5   84.6 -> 62.3
 //         5 / 15 heads  4500 rows  15.3 -> 15.9   18.9 -> 18.2   25.8 -> 23.8   70.3 -> 54.6
 //                       6000 rows  16.1 -> 16.5   21.3 -> 18.8   31.2 -> 25.7   94.2 -> 60.6
-//         1 / 3 heads   6000 rows  21.4 -> 18.1   25.4 -> 20.6   34.9 -> 26.1   89.8 -> 56.8
+//         1 / 3 heads   4500 rows  18.9 -> 16.7   21.7 -> 20.0   29.3 -> 24.0   72.8 -> 48.0
 //   fp32  8 / 32 heads  4512 rows  18.1 -> 16.6   22.5 -> 23.0   32.5 -> 35.0   93.0 -> 106.8
 //                       6016 rows  19.0 -> 16.9   24.9 -> 23.7   36.8 -> 36.0  112.8 -> 111.0
-// (from 6000 rows on the worst of 7 head counts x 8 histories x 2 precisions: 66.2 -> 68.7, fp32, 8 / 32
-// heads, 7008 rows past 8128, whose ranges come out uneven).
-static constexpr int64_t PROMPT_FROM = 6000;
+//         5 / 15 heads  4500 rows  18.5 -> 17.3   23.6 -> 22.9   32.8 -> 33.1   93.6 -> 95.0
+// and past 0 / 100 / 250 / 499, bf16:
+//         5 / 15 heads  5010 rows  15.8 -> 14.8   15.6 -> 15.4   17.0 -> 16.2   17.4 -> 16.9
+//         8 / 32 heads  5024 rows  14.4 -> 15.1   15.0 -> 15.1   15.1 -> 15.6   16.7 -> 17.0
+//                       5504 rows  15.2 -> 14.9   15.7 -> 15.2   16.0 -> 15.8   17.4 -> 17.2
+// (The worst of 7 head counts x 12 histories x 2 precisions on the near side of these lines: fp32, 4 / 12
+// heads, 4500 rows past 2000 26.0 -> 27.2, and 8 / 32 heads, 7008 rows past 8128 66.2 -> 68.7, whose ranges
+// come out uneven.)
+static int64_t prompt_from(int64_t rows, int past) {  // rows of one KV head
+  return rows < 900 ? 5500 : past < 500 ? 5000 : 4500;
+}
 // These kernels look every history token up in the tile table, where the frame-chunk kernel walks the
 // tiles there are and clamps each to its rows: they run only where the host copy of the table shows a tile
 // for each token below past (well under 1 ns per tile and call).
@@ -546,9 +556,10 @@ static int64_t prompt_images(const dkv_attn_args& a) {
   return (int64_t)a.heads * (((int64_t)a.past + a.nq + TILE - 1) / TILE) * prompt_image_bytes(a.precision);
 }
 static bool prompt_route(const dkv_attn_args& a) {
-  return a.path == 0 && a.splits <= 0 && !a.step && (int64_t)a.q_heads * a.nq >= PROMPT_FROM &&
-         (int64_t)(a.q_heads / a.heads) * a.nq >= PROMPT_ROWS &&
-         prompt_images(a) <= PROMPT_MAX_IMAGES && table_covers(a);
+  const int64_t rows = (int64_t)(a.q_heads / a.heads) * a.nq;
+  if (a.path != 0 || a.splits > 0 || a.step || rows < PROMPT_ROWS || rows * a.heads < prompt_from(rows, a.past))
+    return false;
+  return prompt_images(a) <= PROMPT_MAX_IMAGES && table_covers(a);
 }
 
 static PromptPlan make_prompt_plan(const dkv_attn_args& a) {

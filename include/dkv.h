@@ -211,10 +211,10 @@ int64_t dkv_attend_workspace_bytes(const dkv_attn_args* args);
 /* Fused packed-history causal GQA attention. Replaces GPUCache.attend's
  * packed_attention launch (src/gpu_cache.py:96-104, src/gpu_kernels.py:71-105).
  * Frames, candidate batches and decode steps run a split-history MFMA kernel
- * (path 0/2); long chunks (path 0, 6000 query rows or more over all Q heads, no
- * step pair, no explicit split count, and no history or a tiles_host that covers
- * it) unpack the keys once and run a causal MFMA kernel over ranges of them (three
- * launches);
+ * (path 0/2); long chunks (path 0 with some 5000 query rows or more over all Q
+ * heads, no step pair, no explicit split count, and no history or a tiles_host that
+ * covers it) unpack the keys once and run a causal MFMA kernel over ranges of them
+ * (three launches);
  * path 3 runs short chunks (at most 16 query rows per KV head, e.g. decode
  * steps) on a kernel with two waves per 64-key tile. A merge kernel combines
  * the history splits of either in a second launch.

@@ -261,25 +261,28 @@ def test_long_chunks_need_a_table_that_covers_their_history(precision):
         assert need(bad) == need(bad, path=2), change
 
 
-@pytest.mark.parametrize('heads,q_heads,nq,long', [
-    (8, 32, 187, False), (8, 32, 188, True), (5, 15, 399, False), (5, 15, 400, True), (1, 3, 1999, False),
-    (1, 3, 2000, True), (60, 60, 255, False), (60, 60, 256, True),
+@pytest.mark.parametrize('heads,q_heads,nq,always,past_some', [
+    (8, 32, 171, False, False), (8, 32, 172, True, True), (5, 15, 333, False, True), (5, 15, 334, True, True),
+    (5, 15, 300, False, True), (5, 15, 299, False, False), (6, 18, 299, False, False), (1, 3, 1666, False, True),
+    (1, 3, 1667, True, True), (60, 60, 255, False, False), (60, 60, 256, True, True),
 ])
 @pytest.mark.parametrize('precision', [0, 1])
-def test_long_chunk_route_starts_where_it_is_faster(heads, q_heads, nq, long, precision):
-    """From 6000 query rows over all Q heads, and 256 per KV head, at any history; below, the plan of path 2
-    (at 4500 rows and short histories the long-chunk kernels were up to 9% slower)."""
+def test_long_chunk_route_starts_where_it_is_faster(heads, q_heads, nq, always, past_some, precision):
+    """From 5500 query rows over all Q heads, and 256 per KV head, at any history; where a KV head has 900, from
+    5000, and from 4500 if 500 tokens are past. Below, the plan of path 2 (at 4500 rows of 8 KV heads, or without
+    history, the long-chunk kernels were up to 9% slower)."""
     lib = _lib.load()
-    for past in (0, 640, 20032):
-        arr = host_tiles([64] * (past // 64))
+    for past in (0, 499, 500, 640, 20032):
+        tiles = (past + 63) // 64
+        arr = host_tiles([64] * tiles)
         need = {}
         for path in (0, 2):
-            a = attn(past=past, n_tiles=past // 64, arena=4096, tiles=4096, heads=heads, q_heads=q_heads, nq=nq,
+            a = attn(past=past, n_tiles=tiles, arena=4096, tiles=4096, heads=heads, q_heads=q_heads, nq=nq,
                      precision=precision, path=path)
             if past:
                 a.tiles_host = ctypes.addressof(arr)
             need[path] = lib.dkv_attend_workspace_bytes(ctypes.byref(a))
-        assert (need[0] != need[2]) == long
+        assert (need[0] != need[2]) == (past_some if past >= 500 else always), past
 
 
 def test_long_chunk_workspace_is_bounded():
