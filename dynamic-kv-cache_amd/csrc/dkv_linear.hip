@@ -621,8 +621,9 @@ __global__ void __launch_bounds__(256, 3) linear_tile_kernel(const LinearArgs a)
 }
 
 // Q/K/V of many rows, ending in dkv_rope_pack's work as linear_rope_kernel does: the 960-wide decoder's
-// launch at 1000 rows 12.6 us instead of 10.4 + 4.3. A whole layer past 640 in graph replays, two launches
-// -> one: 380 rows 64.6 -> 63.4 us, 512 rows 71.1 -> 69.9, 700 rows 77.5 -> 75.5, 1000 rows 81.7 -> 79.0.
+// launch at 1000 rows 12.6 us instead of 10.4 + 4.3. A whole eager layer past 640, recorded in a HIP graph to
+// time it, two launches -> one: 380 rows 64.6 -> 63.4 us, 512 rows 71.1 -> 69.9, 700 rows 77.5 -> 75.5, 1000
+// rows 81.7 -> 79.0. (Layers of so many rows under graph steps keep the two launches.)
 template <int OPS>
 __global__ void __launch_bounds__(256, 3) linear_tile_rope_kernel(const LinearArgs a, const RopeArgs rope) {
   tile_body<EPI_ROPE, OPS>(a, rope);

@@ -551,10 +551,10 @@ class GPUCache(_CacheBase):
 
         `segments` (optional) lists chunk boundaries [0, b1, ..., nq] for a block-diagonal batch of
         independent continuations that share the history, e.g. QA candidates. `path` is 'auto' (the
-        frame-chunk MFMA kernel, decode steps included, and the long-chunk kernels for prompts of
-        several hundred tokens), 'mfma' (the frame-chunk kernel), 'short' (the short-chunk kernel, at
-        most 16 query rows per KV head) or 'vector'; `precision` overrides the cache's 'bf16' / 'fp32'
-        setting for this call.
+        frame-chunk MFMA kernel, decode steps included, and, unless `as_replayed` is set, the
+        long-chunk kernels for prompts of several hundred tokens), 'mfma' (the frame-chunk kernel),
+        'short' (the short-chunk kernel, at most 16 query rows per KV head) or 'vector'; `precision`
+        overrides the cache's 'bf16' / 'fp32' setting for this call.
         """
         if precision is None:
             precision = self.precision
